@@ -170,6 +170,7 @@ __host__ __device__ inline void shoup_wq(uint32_t wq[27], const uint32_t rem[24]
 // the q*p terms.
 template <class P>
 struct F753 {
+    using params = P;
     using elem_t = E753;
     using tw_t = TW753;
     static constexpr int LIMBS = 24;

@@ -23,7 +23,7 @@ namespace gsn {
 template <int FID>
 struct Collector {
     using F = typename FieldInfo<FID>::Dev;
-    std::map<std::tuple<int, int, int, int>, std::vector<PassJob<F>>> by_key;  // (level, r, w, e)
+    std::map<std::tuple<int, int, int, int, int>, std::vector<PassJob<F>>> by_key;  // (level, r, w, e, kind)
 
     void add(const PlanImpl<FID> &plan, const void *in, void *out, void *ws0, void *ws1)
     {
@@ -31,11 +31,11 @@ struct Collector {
         plan.make_jobs(in, out, ws0, ws1, jobs);
         for (size_t lvl = 0; lvl < jobs.size(); ++lvl) {
             const PassCfg &c = plan.cfg[lvl];
-            // 753-bit tiles take their shape at run time: one group per level
-            // and workgroup size (tile class)
-            const auto key = FieldInfo<FID>::Dev::LIMBS > 1
-                                 ? std::make_tuple((int)lvl, t753_log_tile(c), 0, 1)
-                                 : std::make_tuple((int)lvl, c.log_r, c.log_w, c.log_e);
+            // the vector kernels' 753-bit tiles take their shape at run time:
+            // one group per level and workgroup size (tile class)
+            const auto key = FieldInfo<FID>::Dev::LIMBS > 1 && !c.kind
+                                 ? std::make_tuple((int)lvl, t753_log_tile(c), 0, 1, 0)
+                                 : std::make_tuple((int)lvl, c.log_r, c.log_w, c.log_e, c.kind);
             by_key[key].push_back(jobs[lvl]);
         }
     }
@@ -47,7 +47,8 @@ struct Collector {
             Group g;
             g.field = FID;
             g.level = std::get<0>(kv.first);
-            g.cfg = {std::get<1>(kv.first), std::get<2>(kv.first), std::get<3>(kv.first)};
+            g.cfg = {std::get<1>(kv.first), std::get<2>(kv.first), std::get<3>(kv.first),
+                     std::get<4>(kv.first)};
             for (size_t i = 0; i < jobs.size(); ++i) {
                 jobs[i].first_tile = (uint32_t)g.host_tiles.size();
                 g.host_tiles.insert(g.host_tiles.end(), jobs[i].num_tiles, (uint32_t)i);
@@ -135,7 +136,7 @@ size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count)
     size_t bytes = 0;
     for (size_t i = 0; i < count; ++i) {
         const std::vector<PassCfg> v = choose_passes(items[i].field, items[i].log_n, true);
-        const int nbuf = v.size() >= 3 ? 2 : (v.size() == 2 ? 1 : 0);
+        const int nbuf = schedule_buffers(v);
         bytes += (size_t)nbuf * ((size_t)1 << items[i].log_n) * element_bytes(items[i].field);
         bytes = (bytes + 255) & ~(size_t)255;
     }
@@ -156,8 +157,7 @@ int build_batch(BatchImpl &b, const gsn_batch_item *items, size_t count, int use
         GSN_TRY(cached_plan(&plans[i], it.field, it.log_n, it.omega, it.inverse, true));
         const size_t eb = element_bytes(it.field);
         const size_t n = (size_t)1 << it.log_n;
-        const int P = plans[i]->num_passes;
-        const int nbuf = P >= 3 ? 2 : (P == 2 ? 1 : 0);
+        const int nbuf = plans[i]->workspace_buffers;
         ws_off[i] = ws_bytes;
         ws_bytes += (size_t)nbuf * n * eb;
         ws_bytes = (ws_bytes + 255) & ~(size_t)255;

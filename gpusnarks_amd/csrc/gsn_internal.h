@@ -50,6 +50,7 @@ struct PlanBase {
     unsigned log_n = 0;
     int inverse = 0;
     int num_passes = 0;
+    int workspace_buffers = 0;  // buffers of n elements an execution of a power-of-two plan needs
     bool batch_mode = false;  // schedule of the batch table (fused launches)
     size_t device_bytes = 0;
     std::mutex host_mutex;  // serialises the host entry point's buffer

@@ -35,6 +35,9 @@ struct PassArgs {
     uint32_t col_shift;   // column table index = exponent << col_shift
     uint32_t pass_shift;  // pass table exponent = (r * k) << pass_shift
     uint32_t lo_bits;     // two-level pass table split (0: one table)
+    // 753-bit matrix passes (matrix753_kernels.h): row stride, folded digit,
+    // last and first digit (all log2)
+    uint32_t log_s, log_g, log_np, log_n1;
     uint32_t tw_stride;   // 753-bit: quads per plane of the pass's step table (records + 1)
     uint32_t flags;
     typename F::tw_t scale;
@@ -50,11 +53,23 @@ struct PassJob {
     uint32_t num_tiles;
 };
 
-// One Stockham pass: radix 2^log_r over 2^log_w columns per workgroup with
-// radix-2^log_e register steps.
+// One pass: radix 2^log_r over 2^log_w columns per workgroup with
+// radix-2^log_e register steps.  kind 0 is a Stockham pass of the vector
+// kernels; the others are the 753-bit matrix passes.
+enum : int { MAT_FIRST = 1, MAT_MID = 2, MAT_LAST = 3, MAT_MID2 = 4 };
 struct PassCfg {
     int log_r, log_w, log_e;
+    int kind = 0;
 };
+
+// Workspace buffers of n elements a schedule needs: Stockham passes write
+// another buffer than they read; matrix passes between the first and the
+// last work in place.
+template <class Passes>
+int schedule_buffers(const Passes &v)
+{
+    return v.size() <= 1 ? 0 : v.size() == 2 || v[0].kind ? 1 : 2;
+}
 
 // 753-bit tiles: at most 2^10 elements (99 KiB of LDS, plus up to 56 KiB of
 // staged twiddles).  A tile of 2^t elements runs on a workgroup of 2^(t-1)
@@ -73,6 +88,21 @@ void launch_pass(const PassJob<F> &job, const PassCfg &cfg, hipStream_t stream);
 template <class F>
 void launch_pass_multi(const PassJob<F> *d_jobs, const uint32_t *d_tile_job, uint32_t total_tiles, const PassCfg &cfg,
                        hipStream_t stream);
+
+// The matrix passes (matrix753_*.hip): kinds MAT_*, compiled tile shapes.
+constexpr bool mat_supported(const PassCfg &c)
+{
+    return c.log_e == 1 && c.log_r >= (c.kind == MAT_MID ? 4 : 5) && c.log_r <= 6 && c.log_w == 5;
+}
+template <class F>
+void launch_mat(const PassJob<F> &single, const PassJob<F> *d_jobs, const uint32_t *d_tile_job, uint32_t grid,
+                const PassCfg &cfg, hipStream_t stream);
+// Their byte matrices (build_mat753_kernel); scale null: none.
+constexpr uint32_t MAT_BYTES = 9216;  // one twiddle's matrix: 3 x 3 blocks of 1 KiB
+template <class F>
+void launch_build_mat753(uint4 *out, uint32_t entries, bool fold, const E753 *hi, const TW753 *lo, uint32_t h,
+                         uint32_t log_n, uint32_t log_y, uint64_t mul, uint64_t add, bool pair, const TW753 *scale,
+                         hipStream_t stream);
 
 // gsn_debug_clock_ghz's kernel (kernels_mnt6.hip)
 void launch_clock_probe(unsigned long long *spans, E753 *sink, unsigned blocks, int iters, hipStream_t stream);

@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -112,45 +113,89 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
     return v;
 }
 
+// Matrix passes of a 753-bit transform (matrix753_kernels.h); empty where the
+// vector kernels stay.  Radices of 2^4 .. 2^6 in tiles of 32 columns, the
+// first and the last at least 2^5 (their columns are k1 and jP): three
+// passes from 2^14, four from 2^19 to 2^24.  Where the line lies, time alone
+// on one box, matrix against vector: 2^15 50 / 57 us, 2^16 68 / 60, 2^17
+// 79 / 76, 2^18 99 / 126, 2^19 136 / 249, 2^20 285 / 515, 2^22 1210 / 2280:
+// a transform of 2^16 or 2^17 leaves most of the chip without a tile of
+// 2^11.  Batches fill it, so there everything from 2^15 goes this way (64
+// ragged transforms: 986 us; 998 with 2^14 too, 1031 from 2^16, 1248 with
+// none below 2^18).
+static std::vector<PassCfg> matrix_passes(int field, unsigned L, bool batch)
+{
+    static const int R[][4] = {{5, 5, 5},    {5, 6, 5},    {6, 5, 6},    {6, 6, 6},    {5, 5, 4, 5},
+                               {5, 5, 5, 5}, {6, 5, 5, 5}, {6, 5, 5, 6}, {6, 6, 5, 6}, {6, 6, 6, 6}};
+    std::vector<PassCfg> v;
+    if (field == GSN_FIELD_FP32 || L < 15 || L > 24 || (!batch && (L == 16 || L == 17)))
+        return v;
+    const int *r = R[L - 15], P = r[3] ? 4 : 3;
+    for (int i = 0; i < P; ++i)
+        v.push_back({r[i], 5, 1, i == 0 ? MAT_FIRST : i == P - 1 ? MAT_LAST : i == P - 3 ? MAT_MID2 : MAT_MID});
+    return v;
+}
+
 namespace {
 std::mutex g_tune_mutex;
-std::map<std::pair<int, unsigned>, std::vector<PassCfg>> g_tuned;
-std::map<std::pair<int, unsigned>, std::vector<PassCfg>> g_tuned_batch;  // overrides for fused launches
+using Schedules = std::map<std::pair<int, unsigned>, std::vector<PassCfg>>;
+// schedules set by the program or its own tuning file, and those of the
+// table beside the library; batch: overrides for fused launches
+Schedules g_tuned, g_tuned_batch, g_shipped, g_shipped_batch;
 }  // namespace
 
-int load_schedules(const char *path);
+int load_schedules(const char *path, bool shipped);
 
-// tuning.txt beside the library, or $GSN_TUNING_FILE, read on first use
+// tuning.txt beside the library
+static std::string shipped_table()
+{
+    Dl_info info;
+    if (!dladdr((void *)&shipped_table, &info) || !info.dli_fname)
+        return std::string();
+    const std::string p(info.dli_fname);
+    const size_t slash = p.rfind('/');
+    return (slash == std::string::npos ? std::string(".") : p.substr(0, slash)) + "/tuning.txt";
+}
+
+// the shipped table, or $GSN_TUNING_FILE, read on first use
 static void load_default_schedules()
 {
     const char *env = std::getenv("GSN_TUNING_FILE");
     if (env && *env) {
-        load_schedules(env);
+        load_schedules(env, false);
         return;
     }
-    Dl_info info;
-    if (dladdr((void *)&load_default_schedules, &info) && info.dli_fname) {
-        std::string p(info.dli_fname);
-        const size_t slash = p.rfind('/');
-        p = (slash == std::string::npos ? std::string(".") : p.substr(0, slash)) + "/tuning.txt";
-        std::ifstream f(p);
-        if (f.good())
-            load_schedules(p.c_str());
-    }
+    const std::string p = shipped_table();
+    if (!p.empty() && std::ifstream(p).good())
+        load_schedules(p.c_str(), true);
 }
 
-std::vector<PassCfg> choose_passes(int field, unsigned log_n, bool batch)
+// A schedule that the program set, or read from a table of its own, stands.
+// Elsewhere the matrix passes go first where there are any (matrix_passes),
+// then the shipped table, then the defaults.  matrix = false: the schedule
+// of the vector kernels, which the tuning calls speak of.
+std::vector<PassCfg> choose_passes(int field, unsigned log_n, bool batch, bool matrix)
 {
     static std::once_flag once;
     std::call_once(once, load_default_schedules);
     std::lock_guard<std::mutex> lk(g_tune_mutex);
+    const std::pair<int, unsigned> key{field, log_n};
+    const std::vector<PassCfg> mat = matrix ? matrix_passes(field, log_n, batch) : std::vector<PassCfg>();
     if (batch) {
-        auto ib = g_tuned_batch.find({field, log_n});
+        auto ib = g_tuned_batch.find(key);
         if (ib != g_tuned_batch.end())
             return ib->second;
+        ib = g_shipped_batch.find(key);
+        if (ib != g_shipped_batch.end())
+            return mat.empty() ? ib->second : mat;
     }
-    auto it = g_tuned.find({field, log_n});
+    auto it = g_tuned.find(key);
     if (it != g_tuned.end())
+        return it->second;
+    if (!mat.empty())
+        return mat;
+    it = g_shipped.find(key);
+    if (it != g_shipped.end())
         return it->second;
     return default_passes(field, log_n);
 }
@@ -179,11 +224,16 @@ static int validate_schedule(int field, unsigned log_n, const std::vector<PassCf
     return GSN_OK;
 }
 
-int set_schedule(int field, unsigned log_n, const std::vector<PassCfg> &v, bool batch = false)
+int set_schedule(int field, unsigned log_n, const std::vector<PassCfg> &v, bool batch = false, bool shipped = false)
 {
     GSN_TRY(validate_schedule(field, log_n, v));
     std::lock_guard<std::mutex> lk(g_tune_mutex);
-    (batch ? g_tuned_batch : g_tuned)[{field, log_n}] = v;
+    if (shipped) {  // loading it again restores what it says
+        (batch ? g_tuned_batch : g_tuned).erase({field, log_n});
+        (batch ? g_shipped_batch : g_shipped)[{field, log_n}] = v;
+    } else {
+        (batch ? g_tuned_batch : g_tuned)[{field, log_n}] = v;
+    }
     return GSN_OK;
 }
 
@@ -192,11 +242,13 @@ void clear_schedules()
     std::lock_guard<std::mutex> lk(g_tune_mutex);
     g_tuned.clear();
     g_tuned_batch.clear();
+    g_shipped.clear();
+    g_shipped_batch.clear();
 }
 
 // "field log_n r,w,e r,w,e ..." per line, "batch field log_n ..." for the
 // schedule of transforms fused into batches; '#' starts a comment
-int load_schedules(const char *path)
+int load_schedules(const char *path, bool shipped)
 {
     std::ifstream f(path);
     if (!f.good())
@@ -230,7 +282,7 @@ int load_schedules(const char *path)
                                                                ": bad pass shape '" + tok + "'");
             v.push_back(c);
         }
-        GSN_TRY(set_schedule(field, log_n, v, batch));
+        GSN_TRY(set_schedule(field, log_n, v, batch, shipped));
     }
     return GSN_OK;
 }
@@ -355,10 +407,12 @@ int PlanImpl<GSN_FIELD_FP32>::build_tables(const fields::Fp32 &w, size_t n)
 template <class Plan, class H, class F, class P>
 static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
 {
-    // every record is w_n^e = hi[e >> h] * lo[e & (2^h - 1)] for e < n/2,
+    // every record is w_n^e = hi[e >> h] * lo[e & (2^h - 1)] for e < n/2
+    // (e < n for matrix passes),
     // computed on the device from hi (canonical residues) and lo (records)
+    const bool mat = plan.cfg[0].kind != 0;
     const unsigned h = (log_n + 1) / 2;
-    const size_t nlo = (size_t)1 << h, nhi = std::max<size_t>(1, (n / 2) >> h);
+    const size_t nlo = (size_t)1 << h, nhi = std::max<size_t>(1, (mat ? n : n / 2) >> h);
     std::vector<TW753> lo(nlo);
     std::vector<E753> hi(nhi);
     H acc = H::one();
@@ -381,6 +435,41 @@ static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
     plan.step_tabs.resize(P_);
     plan.step_nrec.assign(P_, 0);
     unsigned log_ns = 0;
+    if (mat) {
+        plan.mat_tabs.resize(3 * P_);
+        plan.mat_share.resize(P_);
+        const auto build = [&](DeviceBuffer &b, size_t entries, bool fold, unsigned log_y, uint64_t mul, uint64_t add,
+                               bool pair, const TW753 *scale) {
+            GSN_TRY(b.alloc(entries * MAT_BYTES));
+            launch_build_mat753<F>((uint4 *)b.ptr, (uint32_t)entries, fold, (const E753 *)dhi.ptr,
+                                   (const TW753 *)dlo.ptr, h, log_n, log_y, mul, add, pair, scale, 0);
+            return hip_status(hipGetLastError(), "matrix table launch");
+        };
+        const unsigned rp = (unsigned)plan.cfg[P_ - 1].log_r;
+        for (size_t i = 0; i < P_; ++i) {
+            const unsigned r = (unsigned)plan.cfg[i].log_r, g = i ? (unsigned)plan.cfg[i - 1].log_r : 0u;
+            size_t own = i;
+            for (size_t k = 1; k < i; ++k)
+                if (plan.cfg[k].log_r == (int)r && plan.cfg[k - 1].log_r == (int)g)
+                    own = std::min(own, k);
+            plan.mat_share[i] = (int)own;
+            if (own == i)
+                GSN_TRY(build(plan.mat_tabs[3 * i], (((size_t)1 << r) - 1) << g, true, g, 0, 0, false, nullptr));
+            if (i > 0 && i < P_ - 1) {
+                // column factors w_n^(jP k(i-1) N1..N(i-2)); n^-1 on the first
+                GSN_TRY(build(plan.mat_tabs[3 * i + 1], (size_t)1 << (g + rp), false, rp,
+                              (uint64_t)1 << (log_ns - g), 0, false, i == 1 && plan.inverse ? &plan.scale : nullptr));
+                if (i + 2 < P_) {  // the pair (1, 3)
+                    const unsigned r3 = (unsigned)plan.cfg[2].log_r;
+                    GSN_TRY(build(plan.mat_tabs[3 * i + 2], (size_t)2 << (g + r3), false, r3, (uint64_t)1 << rp,
+                                  n >> (g + 1), true, nullptr));
+                }
+            }
+            log_ns += r;
+        }
+        GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+        return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
+    }
     for (size_t i = 0; i < P_; ++i) {
         const unsigned lr = (unsigned)plan.cfg[i].log_r;
         const uint32_t nrec = (uint32_t)((((size_t)1 << lr) - 1) << log_ns);
@@ -743,7 +832,7 @@ int gsn_tuning_get(int field, unsigned log_n, int *shapes, int max_passes, int *
 {
     if (!num_passes)
         return set_error(GSN_ERR_INVALID_ARGUMENT, "num_passes is NULL");
-    const std::vector<PassCfg> v = choose_passes(field, log_n);
+    const std::vector<PassCfg> v = choose_passes(field, log_n, false, false);
     *num_passes = (int)v.size();
     if ((int)v.size() > max_passes || (!shapes && !v.empty()))
         return set_error(GSN_ERR_INVALID_ARGUMENT, "shapes buffer too small");
@@ -768,7 +857,10 @@ int gsn_tuning_load(const char *path)
     if (!path)
         return set_error(GSN_ERR_INVALID_ARGUMENT, "path is NULL");
     (void)choose_passes(GSN_FIELD_FP32, 1);
-    GSN_TRY(load_schedules(path));
+    // the shipped table by name restores the defaults
+    char a[PATH_MAX], b[PATH_MAX];
+    const bool shipped = realpath(path, a) && realpath(shipped_table().c_str(), b) && std::strcmp(a, b) == 0;
+    GSN_TRY(load_schedules(path, shipped));
     clear_plan_cache();
     return GSN_OK;
 }

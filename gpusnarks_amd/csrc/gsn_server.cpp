@@ -136,11 +136,11 @@ int enqueue_single_t(PlanBase *base, const gsn_batch_item &it, Wave *w, hipStrea
         launch_scale<F>((const typename F::elem_t *)it.d_in, (typename F::elem_t *)it.d_out, {}, 1, 0, s);
         return hip_status(hipGetLastError(), "copy launch");
     }
-    const int P = plan.num_passes;
+    const int nbuf = plan.workspace_buffers;
     void *ws0 = nullptr, *ws1 = nullptr;
-    if (P >= 2 && !(ws0 = wave_alloc(w, n * sizeof(typename F::elem_t))))
+    if (nbuf >= 1 && !(ws0 = wave_alloc(w, n * sizeof(typename F::elem_t))))
         return set_error(GSN_ERR_OUT_OF_MEMORY, "wave memory exhausted");
-    if (P >= 3 && !(ws1 = wave_alloc(w, n * sizeof(typename F::elem_t))))
+    if (nbuf >= 2 && !(ws1 = wave_alloc(w, n * sizeof(typename F::elem_t))))
         return set_error(GSN_ERR_OUT_OF_MEMORY, "wave memory exhausted");
     std::vector<PassJob<F>> jobs;
     plan.make_jobs(it.d_in, it.d_out, ws0, ws1, jobs);
@@ -168,7 +168,7 @@ size_t request_bytes(int field, unsigned log_n, bool device)
 {
     const size_t n = (size_t)1 << log_n, eb = element_bytes(field);
     const std::vector<PassCfg> v = choose_passes(field, log_n, true);
-    const int nbuf = v.size() >= 3 ? 2 : (v.size() == 2 ? 1 : 0);
+    const int nbuf = schedule_buffers(v);
     size_t bytes = device ? 0 : align_up(n * eb);
     bytes += align_up((size_t)nbuf * n * eb);
     for (const PassCfg &c : v) {

@@ -6,6 +6,8 @@ namespace gsn {
 template <>
 bool pass_supported<FMnt4>(const PassCfg &c)
 {
+    if (c.kind)
+        return mat_supported(c);
     return c.log_e == 1 && c.log_r >= 1 && c.log_w >= 0 && c.log_r + c.log_w <= T753_LOG_TILE;
 }
 
@@ -32,7 +34,10 @@ template <>
 void launch_pass<FMnt4>(const PassJob<FMnt4> &job, const PassCfg &c, hipStream_t st)
 {
     const size_t grid = ((size_t)1 << (job.a.log_n - c.log_r)) >> c.log_w;
-    launch753(job, nullptr, nullptr, (uint32_t)grid, t753_log_tile(c), st);
+    if (c.kind)
+        launch_mat<FMnt4>(job, nullptr, nullptr, (uint32_t)grid, c, st);
+    else
+        launch753(job, nullptr, nullptr, (uint32_t)grid, t753_log_tile(c), st);
 }
 
 template <>
@@ -40,7 +45,10 @@ void launch_pass_multi<FMnt4>(const PassJob<FMnt4> *jobs, const uint32_t *tile_j
                              const PassCfg &c, hipStream_t st)
 {
     PassJob<FMnt4> unused{};
-    launch753(unused, jobs, tile_job, total_tiles, t753_log_tile(c), st);
+    if (c.kind)
+        launch_mat<FMnt4>(unused, jobs, tile_job, total_tiles, c, st);
+    else
+        launch753(unused, jobs, tile_job, total_tiles, t753_log_tile(c), st);
 }
 
 template <>

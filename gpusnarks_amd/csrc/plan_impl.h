@@ -103,6 +103,10 @@ struct PlanImpl final : PlanBase {
     // 753-bit, per pass: step table of Ns (2^r - 1) records in 14 planes
     std::vector<DeviceBuffer> step_tabs;
     std::vector<uint32_t> step_nrec;
+    // 753-bit matrix passes, per pass: folded, column and fixed matrices; a
+    // pass whose folded ones equal another's has the owner in mat_share
+    std::vector<DeviceBuffer> mat_tabs;
+    std::vector<int> mat_share;
     // 32-bit, per pass: column table w_R^x (x < R) and pass table in units
     // of w_{Ns R} -- direct, or hi/lo halves of a two-level split
     std::vector<DeviceBuffer> col_tabs, pass_tabs, pass_los, pass_as;
@@ -118,6 +122,7 @@ struct PlanImpl final : PlanBase {
         const size_t n = (size_t)1 << log_n;
         cfg = choose_passes(FID, log_n, batch_mode);
         num_passes = (int)cfg.size();
+        workspace_buffers = schedule_buffers(cfg);
         for (const PassCfg &c : cfg)
             if (!pass_supported<F>(c))
                 return set_error(GSN_ERR_INVALID_ARGUMENT, "no kernel for the pass configuration");
@@ -126,19 +131,16 @@ struct PlanImpl final : PlanBase {
             return GSN_OK;
         GSN_TRY(build_tables(w, n));
         device_bytes = 0;
-        for (auto *v : {&col_tabs, &pass_tabs, &pass_los, &pass_as, &step_tabs})
+        for (auto *v : {&col_tabs, &pass_tabs, &pass_los, &pass_as, &step_tabs, &mat_tabs})
             for (auto &b : *v)
                 device_bytes += b.bytes;
         return GSN_OK;
     }
 
-    // workspace buffers an execution needs (0, 1 or 2 of n elements)
-    int workspace_buffers() const { return cfg.size() >= 3 ? 2 : (cfg.size() == 2 ? 1 : 0); }
-
     int ensure_scratch()
     {
         const size_t bytes = ((size_t)1 << log_n) * sizeof(elem);
-        for (int i = 0; i < workspace_buffers(); ++i)
+        for (int i = 0; i < workspace_buffers; ++i)
             GSN_TRY(scratch[i].alloc(bytes));
         return GSN_OK;
     }
@@ -152,7 +154,8 @@ struct PlanImpl final : PlanBase {
     int build_tables(const H &w, size_t n);
 
     // Pass jobs for in -> out with workspace ws[0..1]: buffer i (0 < i < P)
-    // alternates ws[0], ws[1], so no pass reads the buffer it writes.
+    // alternates ws[0], ws[1], so no pass reads the buffer it writes; matrix
+    // passes between the first and the last work in place in ws[0].
     void make_jobs(const void *in, void *out, void *ws0, void *ws1, std::vector<PassJob<F>> &jobs) const
     {
         jobs.resize(cfg.size());
@@ -164,7 +167,8 @@ struct PlanImpl final : PlanBase {
     {
         const int P = (int)cfg.size();
         uint32_t log_ns = 0;
-        void *ws[2] = {ws0, ws1};
+        const bool mat = P > 0 && cfg[0].kind;
+        void *ws[2] = {ws0, mat ? ws0 : ws1};
         for (int i = 0; i < P; ++i) {
             const PassCfg &c = cfg[i];
             PassJob<F> jb{};
@@ -179,6 +183,16 @@ struct PlanImpl final : PlanBase {
                 a.tw_pass_a = (const tw *)pass_as[i].ptr;    // nullptr: from the pass table
                 a.lo_bits = pass_lo_bits[i];
                 a.pass_shift = 0;
+            } else if (mat) {
+                // digits of this pass, those after it in the index and the
+                // one before it, as matrix753_kernels.h describes them
+                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]].ptr;
+                a.tw_pass = (const tw *)mat_tabs[3 * i + 1].ptr;
+                a.tw_pass_a = (const tw *)mat_tabs[3 * i + 2].ptr;
+                a.log_s = log_n - log_ns - (uint32_t)c.log_r;
+                a.log_g = i == 0 ? 0u : (uint32_t)cfg[i - 1].log_r;
+                a.log_np = (uint32_t)cfg[P - 1].log_r;
+                a.log_n1 = (uint32_t)cfg[0].log_r;
             } else {
                 // the 753-bit kernel folds the pass twiddles into its step
                 // twiddles, read from the pass's step table
@@ -195,7 +209,8 @@ struct PlanImpl final : PlanBase {
             a.log_ns = log_ns;
             // the inverse's n^-1: for the 753-bit field with two or more
             // passes, on the last pass's inputs (its step-0 records carry it)
-            const uint32_t scale_flag = !IS32 && P >= 2 ? PASS_SCALE_IN : PASS_SCALE;
+            // (a matrix schedule's column factors carry it)
+            const uint32_t scale_flag = mat ? 0u : !IS32 && P >= 2 ? PASS_SCALE_IN : PASS_SCALE;
             a.flags = (i == P - 1) ? (PASS_CANON | (inverse ? scale_flag : 0u)) : 0u;
             a.scale = scale;
             jb.log_r = (uint32_t)c.log_r;
@@ -230,7 +245,7 @@ struct PlanImpl final : PlanBase {
     size_t workspace_bytes() const override
     {
         const size_t one = ((size_t)1 << log_n) * sizeof(elem);
-        const int nb = workspace_buffers();
+        const int nb = workspace_buffers;
         return nb == 0 ? 0 : nb == 1 ? one : ((one + 255) & ~(size_t)255) + one;
     }
 

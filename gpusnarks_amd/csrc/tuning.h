@@ -12,6 +12,6 @@
 namespace gsn {
 
 std::vector<PassCfg> default_passes(int field, unsigned log_n);
-std::vector<PassCfg> choose_passes(int field, unsigned log_n, bool batch = false);
+std::vector<PassCfg> choose_passes(int field, unsigned log_n, bool batch = false, bool matrix = true);
 
 }  // namespace gsn

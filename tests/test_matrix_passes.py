@@ -1,0 +1,154 @@
+"""The 753-bit matrix passes (gpusnarks_amd/csrc/matrix753_kernels.h) restated
+in Python, CPU only: their arithmetic with whole numbers at the ends of its
+ranges, and their digits, twiddle factors and addresses over a small prime
+field against the O(n^2) DFT."""
+import random
+
+import numpy as np
+import pytest
+
+import gpusnarks_amd as g
+
+FIELDS = [g.FIELD_MNT4753_FR, g.FIELD_MNT6753_FR]
+TOP = 1 << 768
+OFFSET = int("80" * 96, 16)
+BIAS, BIAS_ROW0 = (1 << 22) - (1 << 14), 1 << 14
+LIFT = 12400
+
+
+def digits(x):
+    """The signed byte digits of x from its offset form."""
+    return [b - 128 for b in ((x + OFFSET) % TOP).to_bytes(96, "little")]
+
+
+def columns(w, p):
+    cols = []
+    for k in range(96):
+        c = (w << (8 * k)) % p
+        # the kernel centres by the top limb alone
+        cols.append(c - p if (c >> 736) > (p >> 736) // 2 else c)
+    return cols
+
+
+def product(y, w, p):
+    """mat753_mul: column sums from BIAS, four to a limb, one carry chain."""
+    cols, dy = columns(w, p), digits(y)
+    m = np.array([digits(c) for c in cols], dtype=np.int64).T
+    sums = m @ np.array(dy, dtype=np.int64) + BIAS
+    assert sums.min() >= 0 and sums.max() < 1 << 23
+    t = carry = prev = 0
+    for l in range(24):
+        n0, n1 = int(sums[4 * l] + (sums[4 * l + 1] << 8)), int(sums[4 * l + 2] + (sums[4 * l + 3] << 8))
+        assert n0 < 1 << 31 and n1 < 1 << 31
+        n0 += BIAS_ROW0 if l == 0 else 0
+        v = n0 + (((n1 << 16) | (prev >> 16)) & 0xFFFFFFFF) + carry
+        t |= (v & 0xFFFFFFFF) << (32 * l)
+        carry, prev = v >> 32, n1
+    return t - TOP if t >> 767 else t
+
+
+def reduced(x, p):
+    """Mat753::reduce: the quotient from the top limb in single precision."""
+    top = np.float32((p >> 736) + ((p >> 704) & 0xFFFFFFFF) / 2.0 ** 32)
+    xt = (((x + OFFSET) % TOP) >> 736) - 0x80808080
+    q = int(np.rint(np.float32(xt) * np.float32(1.0 / float(top))))
+    return x - q * p
+
+
+@pytest.mark.parametrize("field", FIELDS)
+def test_products_and_bounds(field):
+    p = g.MODULI[field]
+    bound = 6144 * p
+    limit = 2 * bound + 6 * p
+    # the digits' range, the lift and the top limb cover every value
+    assert -OFFSET <= -limit and limit <= (TOP - 1) - OFFSET
+    assert LIFT * p > limit and LIFT * p + limit < TOP
+    rng = random.Random(field)
+    ws = [0, 1, p - 1, p // 2, p // 2 + 1] + [rng.randrange(p) for _ in range(6)]
+    ys = [0, 1, -1, limit, -limit, 2 * bound, -2 * bound] + [rng.randrange(-limit, limit) for _ in range(6)]
+    # digits all at one end against the signs of the columns' own extremes
+    for w in ws:
+        cols = columns(w, p)
+        assert all(abs(c) <= p // 2 + (p >> 15) for c in cols)
+        for y in ys + [sum((-128 if c > 0 else 127) << (8 * k) for k, c in enumerate(cols[:95]))]:
+            t = product(y, w, p)
+            assert (t - y * w) % p == 0 and abs(t) <= bound + (96 * 128 * p >> 15)
+    for x in ys + [k * p // 2 + d for k in range(-24000, 24000, 997) for d in (-1, 0, 1)]:
+        if abs(x) <= limit:
+            assert abs(reduced(x, p)) <= 0.52 * p
+
+
+# ------------------------------------------------------------ the passes
+
+P, G = 3 * 2 ** 30 + 1, 5
+
+
+def column_dft(col, r, log_g, kap, table):
+    """Steps of one column: in-place decimation in time over positions, the
+    twiddle of step s from entry ((2^s - 1) << log_g) + (kap << s) + kk."""
+    R = 1 << r
+    v = [col[int(format(i, "0%db" % r)[::-1], 2)] for i in range(R)]
+    for s in range(r):
+        for i in range(R):
+            if not i & (1 << s):
+                kk = i & ((1 << s) - 1)
+                t = v[i | (1 << s)] * table[((1 << s) - 1 << log_g) + (kap << s) + kk] % P
+                v[i], v[i | (1 << s)] = (v[i] + t) % P, (v[i] - t) % P
+    return v
+
+
+def fold_table(w, n, r, log_g):
+    out = []
+    for i in range(((1 << r) - 1) << log_g):
+        s = ((i >> log_g) + 1).bit_length() - 1
+        rest = i - (((1 << s) - 1) << log_g)
+        gi, kk = rest >> s, rest & ((1 << s) - 1)
+        out.append(pow(w, (gi + (kk << log_g)) * (n >> (log_g + s + 1)), P))
+    return out
+
+
+@pytest.mark.parametrize("radices", [(2, 2, 2), (1, 3, 2), (3, 2, 3), (2, 1, 2, 2), (2, 2, 1, 3), (1, 2, 3, 1)])
+def test_passes_match_dft(radices):
+    log_n, num = sum(radices), len(radices)
+    n = 1 << log_n
+    w = pow(G, (P - 1) >> log_n, P)
+    rng = random.Random(log_n * num)
+    a = [rng.randrange(P) for _ in range(n)]
+    want = [sum(x * pow(w, j * k, P) for j, x in enumerate(a)) % P for k in range(n)]
+    buf, rp, n1 = list(a), radices[-1], radices[0]
+    out = [None] * n
+    log_ns = 0
+    for i, r in enumerate(radices):
+        R, log_g = 1 << r, radices[i - 1] if i else 0
+        fold = fold_table(w, n, r, log_g)
+        if i < num - 1:
+            log_s = log_n - log_ns - r
+            for blk in range(n >> r):  # one column at a time
+                log_hi = log_n - r - log_s - log_g
+                p, lo = blk >> log_s, blk & ((1 << log_s) - 1)
+                kap = p >> log_hi if i else 0
+                pre = ((p & ((1 << log_hi) - 1)) << log_g) | kap if i else 0
+                base = (pre << (log_s + r)) + lo
+                col = [buf[base + (row << log_s)] for row in range(R)]
+                if i and i == num - 3:  # the pair (1, 3), on both halves of step 0
+                    e = kap * (lo >> rp) << rp
+                    col = [x * pow(w, e, P) % P for x in col]
+                v = column_dft(col, r, log_g, kap, fold)
+                if i:  # the column factor of jP
+                    e = (lo & ((1 << rp) - 1)) * kap << (log_ns - log_g)
+                    v = [x * pow(w, e, P) % P for x in v]
+                for row in range(R):
+                    buf[base + (row << log_s)] = v[row]
+        else:
+            for blk in range(n >> r):
+                rev, k1 = blk >> n1, blk & ((1 << n1) - 1)
+                log_k = log_n - n1 - r - log_g
+                kap = rev >> log_k
+                mid = ((rev & ((1 << log_k) - 1)) << log_g) | kap if log_k else rev
+                at = k1 * (n >> n1) + (mid << r)
+                v = column_dft(buf[at:at + R], r, log_g, kap, fold)
+                for row in range(R):
+                    assert out[(row << (log_n - r)) + (rev << n1) + k1] is None
+                    out[(row << (log_n - r)) + (rev << n1) + k1] = v[row]
+        log_ns += r
+    assert out == want
