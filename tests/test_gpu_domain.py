@@ -295,6 +295,34 @@ def test_mixed_radix_matches_oracle(orc, field, n1, a):
     assert np.array_equal(e.download(x.shape), x)
 
 
+# The odd passes' 64-column wavefronts start at a = 6: both sides of it, each
+# radix as the only, the first, a middle and the last pass.
+@pytest.mark.parametrize("field,n1,a", [(g.FIELD_MNT4753_FR, 3, 6), (g.FIELD_MNT4753_FR, 5, 7),
+                                        (g.FIELD_MNT4753_FR, 7, 6), (g.FIELD_MNT4753_FR, 21, 5),
+                                        (g.FIELD_MNT4753_FR, 25, 6), (g.FIELD_MNT6753_FR, 35, 6),
+                                        (g.FIELD_MNT6753_FR, 49, 6), (g.FIELD_MNT6753_FR, 63, 6),
+                                        (g.FIELD_MNT6753_FR, 245, 8)])
+def test_mixed_radix_column_groups(orc, field, n1, a):
+    n = n1 << a
+    p, L = g.MODULI[field], g.NLIMBS[field]
+    x = residues(field, n, 0x6C0 + n)
+    # sums of q equal extremes: all of one column p - 1, another alternating
+    top = np.frombuffer((p - 1).to_bytes(4 * L, "little"), dtype=np.uint32)
+    x[1::1 << a] = top
+    x[2::2 << a] = top
+    x[3::1 << a] = 0
+    w2, w1 = mixed_roots(field, n1, a)
+    say("mixed radix columns field", field, "n1", n1, "a", a)
+    want = orc.mixed_fft(field, x, n1, w2, w1)
+    d, e = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+    g.Plan.mixed(field, n).execute(d.ptr, e.ptr)
+    g.synchronize()
+    assert np.array_equal(e.download(x.shape), want)
+    g.Plan.mixed(field, n, inverse=True).execute(e.ptr, e.ptr)
+    g.synchronize()
+    assert np.array_equal(e.download(x.shape), x)
+
+
 def test_mixed_radix_mnt4_largest():
     """MNT4-753 Fr at n = 2^15 * 525 (17 million points, past its 2-adicity
     by a factor 1050): the inverse undoes the forward, and X_0 = sum x."""
