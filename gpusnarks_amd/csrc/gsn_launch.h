@@ -55,8 +55,9 @@ struct PassJob {
 
 // One pass: radix 2^log_r over 2^log_w columns per workgroup with
 // radix-2^log_e register steps.  kind 0 is a Stockham pass of the vector
-// kernels; the others are the 753-bit matrix passes.
-enum : int { MAT_FIRST = 1, MAT_MID = 2, MAT_LAST = 3, MAT_MID2 = 4 };
+// kernels; the others are the 753-bit matrix passes, of which MAT_DENSE
+// (dense753.hip) are Stockham passes, too.
+enum : int { MAT_FIRST = 1, MAT_MID = 2, MAT_LAST = 3, MAT_MID2 = 4, MAT_DENSE = 5 };
 struct PassCfg {
     int log_r, log_w, log_e;
     int kind = 0;
@@ -68,7 +69,7 @@ struct PassCfg {
 template <class Passes>
 int schedule_buffers(const Passes &v)
 {
-    return v.size() <= 1 ? 0 : v.size() == 2 || v[0].kind ? 1 : 2;
+    return v.size() <= 1 ? 0 : v.size() == 2 || (v[0].kind && v[0].kind != MAT_DENSE) ? 1 : 2;
 }
 
 // 753-bit tiles: at most 2^10 elements (99 KiB of LDS, plus up to 56 KiB of

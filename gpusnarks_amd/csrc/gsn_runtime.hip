@@ -24,6 +24,7 @@
 #include <string>
 #include <vector>
 
+#include "dense753.h"
 #include "device_field.h"
 #include "gpusnarks.h"
 #include "gsn_internal.h"
@@ -113,21 +114,35 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
     return v;
 }
 
-// Matrix passes of a 753-bit transform (matrix753_kernels.h); empty where the
-// vector kernels stay.  Radices of 2^4 .. 2^6 in tiles of 32 columns, the
-// first and the last at least 2^5 (their columns are k1 and jP): three
-// passes from 2^14, four from 2^19 to 2^24.  Where the line lies, time alone
-// on one box, matrix against vector: 2^15 50 / 57 us, 2^16 68 / 60, 2^17
-// 79 / 76, 2^18 99 / 126, 2^19 136 / 249, 2^20 285 / 515, 2^22 1210 / 2280:
-// a transform of 2^16 or 2^17 leaves most of the chip without a tile of
-// 2^11.  Batches fill it, so there everything from 2^15 goes this way (64
-// ragged transforms: 986 us; 998 with 2^14 too, 1031 from 2^16, 1248 with
-// none below 2^18).
+// Matrix passes of a 753-bit transform; empty where the vector kernels stay.
+//
+// Alone, 2^10 .. 2^15: dense passes (dense753.hip), whose work grows as n R
+// and which need 32 columns.  Against the vector kernels, with other radices
+// in brackets, time on one box: 2^10 16 / 35 us, 2^11 18 / 40, 2^12 20 / 41
+// (three passes 22), 2^13 23 / 44 (2^7 2^6 25), 2^14 26 / 48 (2^7 2^7 30),
+// 2^15 39 / 57 (one column group a block 40, the passes below 50), 2^16 73 /
+// 60.
+//
+// Others: passes of matrix753_kernels.h.  Radices of 2^4 .. 2^6 in tiles of
+// 32 columns, the first and the last at least 2^5 (their columns are k1 and
+// jP): three passes from 2^15, four from 2^19 to 2^24.  Where the line lies,
+// matrix against vector: 2^16 68 / 60 us, 2^17 79 / 76, 2^18 99 / 126, 2^19
+// 136 / 249, 2^20 285 / 515, 2^22 1210 / 2280: a transform of 2^16 or 2^17
+// leaves most of the chip without a tile of 2^11.  Batches fill it, so there
+// everything from 2^15 goes this way (64 ragged transforms: 986 us; 998 with
+// 2^14 too, 1031 from 2^16, 1248 with none below 2^18).
 static std::vector<PassCfg> matrix_passes(int field, unsigned L, bool batch)
 {
     static const int R[][4] = {{5, 5, 5},    {5, 6, 5},    {6, 5, 6},    {6, 6, 6},    {5, 5, 4, 5},
                                {5, 5, 5, 5}, {6, 5, 5, 5}, {6, 5, 5, 6}, {6, 6, 5, 6}, {6, 6, 6, 6}};
+    static const int DENSE[][3] = {{5, 5}, {6, 5}, {6, 6}, {4, 4, 5}, {4, 5, 5}, {5, 5, 5}};
     std::vector<PassCfg> v;
+    if (field != GSN_FIELD_FP32 && !batch && L >= 10 && L <= 15) {
+        for (int r : DENSE[L - 10])
+            if (r)
+                v.push_back({r, L == 15 ? 6 : 5, 1, MAT_DENSE});
+        return v;
+    }
     if (field == GSN_FIELD_FP32 || L < 15 || L > 24 || (!batch && (L == 16 || L == 17)))
         return v;
     const int *r = R[L - 15], P = r[3] ? 4 : 3;
@@ -445,6 +460,30 @@ static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
                                    (const TW753 *)dlo.ptr, h, log_n, log_y, mul, add, pair, scale, 0);
             return hip_status(hipGetLastError(), "matrix table launch");
         };
+        if (plan.cfg[0].kind == MAT_DENSE) {
+            for (size_t i = 0; i < P_; ++i) {
+                const unsigned r = (unsigned)plan.cfg[i].log_r;
+                size_t own = 0;
+                while (plan.cfg[own].log_r != (int)r)
+                    ++own;
+                plan.mat_share[i] = (int)own;
+                log_ns += r;
+                DeviceBuffer &mat = plan.mat_tabs[3 * i], &rec = plan.mat_tabs[3 * i + 1];
+                if (own == i)
+                    GSN_TRY(mat.alloc((size_t)MAT_BYTES << r));
+                unsigned next = 0;
+                if (i + 1 < P_) {
+                    next = (unsigned)plan.cfg[i + 1].log_r;
+                    GSN_TRY(rec.alloc(sizeof(TW753) << (log_ns + next)));
+                }
+                // n^-1 on the first pass's records
+                launch_build_dense753<F>((uint4 *)mat.ptr, r, (TW753 *)rec.ptr, log_ns, next, (const E753 *)dhi.ptr,
+                                         (const TW753 *)dlo.ptr, h, log_n,
+                                         i == 0 && plan.inverse ? &plan.scale : nullptr, 0);
+                GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+            }
+            return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
+        }
         const unsigned rp = (unsigned)plan.cfg[P_ - 1].log_r;
         for (size_t i = 0; i < P_; ++i) {
             const unsigned r = (unsigned)plan.cfg[i].log_r, g = i ? (unsigned)plan.cfg[i - 1].log_r : 0u;

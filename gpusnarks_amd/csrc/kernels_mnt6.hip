@@ -1,4 +1,5 @@
 // Pass and table kernels of the 753-bit field MNT6-753 Fr.
+#include "dense753.h"
 #include "ntt_kernels.h"
 
 namespace gsn {
@@ -7,7 +8,7 @@ template <>
 bool pass_supported<FMnt6>(const PassCfg &c)
 {
     if (c.kind)
-        return mat_supported(c);
+        return c.kind == MAT_DENSE ? dense_supported(c) : mat_supported(c);
     return c.log_e == 1 && c.log_r >= 1 && c.log_w >= 0 && c.log_r + c.log_w <= T753_LOG_TILE;
 }
 
@@ -34,7 +35,9 @@ template <>
 void launch_pass<FMnt6>(const PassJob<FMnt6> &job, const PassCfg &c, hipStream_t st)
 {
     const size_t grid = ((size_t)1 << (job.a.log_n - c.log_r)) >> c.log_w;
-    if (c.kind)
+    if (c.kind == MAT_DENSE)
+        launch_dense753<FMnt6>(job, (job.a.flags & PASS_CANON) != 0, st);
+    else if (c.kind)
         launch_mat<FMnt6>(job, nullptr, nullptr, (uint32_t)grid, c, st);
     else
         launch753(job, nullptr, nullptr, (uint32_t)grid, t753_log_tile(c), st);

@@ -103,8 +103,9 @@ struct PlanImpl final : PlanBase {
     // 753-bit, per pass: step table of Ns (2^r - 1) records in 14 planes
     std::vector<DeviceBuffer> step_tabs;
     std::vector<uint32_t> step_nrec;
-    // 753-bit matrix passes, per pass: folded, column and fixed matrices; a
-    // pass whose folded ones equal another's has the owner in mat_share
+    // 753-bit matrix passes, per pass: folded, column and fixed matrices, or
+    // (dense) matrices and the next pass's records; a pass whose first ones
+    // equal another's has the owner in mat_share
     std::vector<DeviceBuffer> mat_tabs;
     std::vector<int> mat_share;
     // 32-bit, per pass: column table w_R^x (x < R) and pass table in units
@@ -168,7 +169,8 @@ struct PlanImpl final : PlanBase {
         const int P = (int)cfg.size();
         uint32_t log_ns = 0;
         const bool mat = P > 0 && cfg[0].kind;
-        void *ws[2] = {ws0, mat ? ws0 : ws1};
+        const bool dense = mat && cfg[0].kind == MAT_DENSE;
+        void *ws[2] = {ws0, mat && !dense ? ws0 : ws1};
         for (int i = 0; i < P; ++i) {
             const PassCfg &c = cfg[i];
             PassJob<F> jb{};
@@ -183,6 +185,10 @@ struct PlanImpl final : PlanBase {
                 a.tw_pass_a = (const tw *)pass_as[i].ptr;    // nullptr: from the pass table
                 a.lo_bits = pass_lo_bits[i];
                 a.pass_shift = 0;
+            } else if (dense) {
+                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]].ptr;
+                a.tw_pass = (const tw *)mat_tabs[3 * i + 1].ptr;
+                a.log_np = i + 1 < P ? (uint32_t)cfg[i + 1].log_r : 0u;
             } else if (mat) {
                 // digits of this pass, those after it in the index and the
                 // one before it, as matrix753_kernels.h describes them
@@ -209,7 +215,7 @@ struct PlanImpl final : PlanBase {
             a.log_ns = log_ns;
             // the inverse's n^-1: for the 753-bit field with two or more
             // passes, on the last pass's inputs (its step-0 records carry it)
-            // (a matrix schedule's column factors carry it)
+            // (a matrix schedule's column factors or records carry it)
             const uint32_t scale_flag = mat ? 0u : !IS32 && P >= 2 ? PASS_SCALE_IN : PASS_SCALE;
             a.flags = (i == P - 1) ? (PASS_CANON | (inverse ? scale_flag : 0u)) : 0u;
             a.scale = scale;

@@ -62,3 +62,28 @@ def test_matrix_passes_match_vector_kernels(field, log_n):
             g.tuning_load(shipped)  # the default routes again
         assert np.array_equal(got, want), (field, log_n, inverse)
         assert np.array_equal(both[0], want) and np.array_equal(both[1], want), (field, log_n, inverse)
+
+
+@pytest.mark.parametrize("field,log_n", [(f, l) for f in (g.FIELD_MNT4753_FR, g.FIELD_MNT6753_FR)
+                                         for l in (10, 11, 12, 13, 14, 15)])
+def test_dense_passes_match_vector_kernels(field, log_n):
+    """Every schedule of the dense passes (2^10 to 2^15 alone), out of place
+    and in place, two executions of one plan back to back."""
+    x = operands(field, log_n, 0xDE5 + log_n)
+    vector = [(7, 0, 1)] * (log_n // 7) + ([(log_n % 7, 2, 1)] if log_n % 7 else [])
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+    for inverse in (False, True):
+        print("dense passes", field, log_n, inverse, flush=True)
+        plan = g.Plan(field, log_n, inverse=inverse)
+        got, again = run(plan, x, in_place=False), run(plan, x[::-1].copy(), in_place=True)
+        plan.close()
+        try:
+            g.tuning_set(field, log_n, vector)
+            plan = g.Plan(field, log_n, inverse=inverse)
+            assert plan.num_passes == len(vector)
+            want, want_again = run(plan, x, in_place=False), run(plan, x[::-1].copy(), in_place=False)
+            plan.close()
+        finally:
+            g.tuning_clear()
+            g.tuning_load(shipped)  # the default routes again
+        assert np.array_equal(got, want) and np.array_equal(again, want_again), (field, log_n, inverse)

@@ -152,3 +152,38 @@ def test_passes_match_dft(radices):
                     out[(row << (log_n - r)) + (rev << n1) + k1] = v[row]
         log_ns += r
     assert out == want
+
+
+@pytest.mark.parametrize("field", FIELDS)
+def test_dense_sums_and_bounds(field):
+    """dense753.hip: column sums of up to 8 terms from 2^17 255, 25 limbs, the
+    quotient from the top two in single precision, four such parts plus 3 p."""
+    p = g.MODULI[field]
+    bias, row0 = 255 << 17, 1 << 17
+    top = np.float32((p >> 736) + ((p >> 704) & 0xFFFFFFFF) / 2.0 ** 32)
+    inv = np.float32(1.0 / float(top))
+    assert 8 * 96 * 2 ** 14 < bias and 2 * p < OFFSET and -2 * p > -OFFSET
+    rng = random.Random(field + 100)
+    for case in range(8):
+        parts, exact = [], 0
+        for _ in range(4):
+            sums, want = np.full(96, bias, dtype=np.int64), 0
+            for _ in range(8):
+                w = rng.choice([0, 1, p - 1, p // 2, p // 2 + 1, rng.randrange(p)])
+                cols = columns(w, p)
+                y = rng.choice([0, 4 * p, -2 * p, 2 * p - 1, rng.randrange(-2 * p, 4 * p)])
+                if case < 2:  # every digit at the end that makes its column largest
+                    y = sum((-128 if (c > 0) != (case == 1) else 127) << (8 * k) for k, c in enumerate(cols[:95]))
+                sums += np.array([digits(c) for c in cols], dtype=np.int64).T @ np.array(digits(y), dtype=np.int64)
+                want += y * w
+            assert sums.min() >= 0 and sums.max() < 1 << 31
+            total = sum(int(s) << (8 * r) for r, s in enumerate(sums)) + row0
+            low, high = total % TOP, (total >> 768) - row0
+            f = np.float32(np.float32(high) * np.float32(2.0 ** 32) + np.float32(low >> 736)) * inv
+            q = int(np.rint(f))
+            part = high * TOP + low - q * p
+            assert abs(part) <= 0.51 * p and (part - want) % p == 0
+            parts.append(part)
+            exact += want
+        y = sum(parts) + 3 * p
+        assert 0 < y < TOP and (y - exact) % p == 0
