@@ -5,7 +5,7 @@
 
 namespace gsn {
 
-// radices and columns per block compiled
+// radices compiled, and columns of a block
 constexpr bool dense_supported(const PassCfg &c)
 {
     return c.log_e == 1 && ((c.log_w == 5 && c.log_r >= 4 && c.log_r <= 6) || (c.log_w == 6 && c.log_r == 5));

@@ -13,45 +13,44 @@
 // factors up to the sign of odd terms:
 //   Y_k, Y_(k+R/2) = S_even +- S_odd,  S = sum z_j w_R^(j k).
 //
-// A block makes outputs k and k + R/2 of G groups of 32 columns; its four
-// wavefronts take a quarter of the terms each, an even and an odd one at a
-// time in their two halves.  It reads R/2 matrices (9216 B) and 32 G R
-// elements once: 123, 245, 490 KB for R = 16, 32, 64 and one group, which at
-// the CU's 64 bytes a clock is 0.8, 1.6, 3.2 us and bounds the pass together
-// with the final product (2.6 us) and the launch (3.5 us); 18 MFMAs per two
-// terms take a quarter of it.  2^10 points, two passes: 16 us, on the vector
-// kernels 35.  The reads grow as n R, so larger transforms go other ways
-// (matrix_passes).
+// KS wavefronts share the terms of outputs k and k + R/2 of 32 columns, an
+// even and an odd term at a time in their two halves; a block is four of
+// them: KS = 4 spreads the least work over the most wavefronts, KS = 2 leaves
+// fewer carry chains and sums between them where there are columns enough
+// (2^15: 36 against 40 us; KS = 1: 48).  KS wavefronts read R/2 matrices
+// (9216 B) and 32 R elements once: 123, 245, 490 KB for R = 16, 32, 64, which
+// at the CU's 64 bytes a clock is 0.8, 1.6, 3.2 us and bounds the pass
+// together with the final product (2.6 us) and the launch (3.5 us); 18 MFMAs
+// per two terms take a quarter of it.  2^10 points, two passes: 16 us, on the
+// vector kernels 35.  The reads grow as n R, so larger transforms go other
+// ways (matrix_passes).
 #include "dense753.h"
 #include "matrix753_kernels.h"
 
 namespace gsn {
 
-// Accumulator start of the wave's even terms: column sums of up to 8 terms
-// (8 * 96 * 2^14 < 2^24) stay positive.  Over the 96 rows it adds
-// 2^17 (2^768 - 1).
-constexpr int DENSE_BIAS = 255 << 17;
-constexpr uint32_t DENSE_BIAS_ROW0 = 1u << 17;
+// Accumulator start of the wave's even terms: column sums of up to 32
+// terms (32 * 96 * 2^14 < 2^26) stay positive.  Over the 96 rows it adds
+// 2^18 (2^768 - 1).
+constexpr int DENSE_BIAS = 255 << 18;
+constexpr uint32_t DENSE_BIAS_ROW0 = 1u << 18;
 
-template <class F, int LOG_R, int G>
+template <class F, int LOG_R, int KS>
 struct DenseWave {
     using P = typename F::params;
     using M = Mat753<P>;
-    static constexpr int R = 1 << LOG_R, ROUNDS = R / 16;
+    static constexpr int R = 1 << LOG_R, ROUNDS = R / (4 * KS);
 
     struct Terms {  // an even and an odd term: matrices and each lane's x_j, x_(j + R/2)
         v4i m[2][9];
-        E753 x0[G], x1[G];
+        E753 x0, x1;
     };
     __device__ __forceinline__ static void load(Terms &t, const PassArgs<F> &a, uint32_t k, size_t col, uint32_t j)
     {
         const int lane = (int)__lane_id();
         const uint32_t log_c = a.log_n - LOG_R;
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            t.x0[g] = F::load(a.in, ((size_t)(j + (lane >> 5)) << log_c) + col + 32 * g);
-            t.x1[g] = F::load(a.in, ((size_t)(j + R / 2 + (lane >> 5)) << log_c) + col + 32 * g);
-        }
+        t.x0 = F::load(a.in, ((size_t)(j + (lane >> 5)) << log_c) + col);
+        t.x1 = F::load(a.in, ((size_t)(j + R / 2 + (lane >> 5)) << log_c) + col);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const gcv4i *m =
@@ -62,31 +61,27 @@ struct DenseWave {
         }
     }
     // x0 + x1 or, for odd k, x0 - x1, as digits
-    __device__ __forceinline__ static void operands(v4i (&b0)[3], v4i (&b1)[3], const E753 &x0, const E753 &x1,
-                                                    uint32_t odd)
+    __device__ __forceinline__ static void operands(v4i (&b0)[3], v4i (&b1)[3], const Terms &t, uint32_t odd)
     {
         const uint32_t mask = 0u - odd;
         E753 z;
         unsigned c = odd;
 #pragma unroll
         for (int i = 0; i < 24; ++i)
-            z.v[i] = __builtin_addc(x0.v[i], x1.v[i] ^ mask, c, &c);
+            z.v[i] = __builtin_addc(t.x0.v[i], t.x1.v[i] ^ mask, c, &c);
         M::digits(b0, b1, M::to_offset(z));
     }
-    __device__ __forceinline__ static void add(v16i (&se)[G][3], v16i (&so)[G][3], const Terms &t, uint32_t odd)
+    __device__ __forceinline__ static void add(v16i (&se)[3], v16i (&so)[3], const Terms &t, uint32_t odd)
     {
+        v4i b0[3], b1[3];
+        operands(b0, b1, t, odd);
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            v4i b0[3], b1[3];
-            operands(b0, b1, t.x0[g], t.x1[g], odd);
+        for (int I = 0; I < 3; ++I)
 #pragma unroll
-            for (int I = 0; I < 3; ++I)
-#pragma unroll
-                for (int J = 0; J < 3; ++J) {
-                    se[g][I] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t.m[0][3 * I + J], b0[J], se[g][I], 0, 0, 0);
-                    so[g][I] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t.m[1][3 * I + J], b1[J], so[g][I], 0, 0, 0);
-                }
-        }
+            for (int J = 0; J < 3; ++J) {
+                se[I] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t.m[0][3 * I + J], b0[J], se[I], 0, 0, 0);
+                so[I] = __builtin_amdgcn_mfma_i32_32x32x32_i8(t.m[1][3 * I + J], b1[J], so[I], 0, 0, 0);
+            }
     }
     // The limbs of S_even + S_odd in the low half of the wave and of
     // S_even - S_odd in the high one (rows as in mat753_mul), reduced to
@@ -117,7 +112,7 @@ struct DenseWave {
                 y.v[l + 1] = __builtin_addc(lo[1], hi[0], carry, &carry);
                 prev = hi[1];
             }
-        // |y| < 8 * 6144 p: the quotient from limbs 23 and 24
+        // |y| < 32 * 6144 p: the quotient from limbs 23 and 24
         const int32_t top = (int32_t)(prev + carry - DENSE_BIAS_ROW0);
         constexpr double TOP = (double)P::MOD[23] + (double)P::MOD[22] / 4294967296.0;
         const float f = ((float)top * 4294967296.0f + (float)y.v[23]) * (float)(1.0 / TOP);
@@ -151,65 +146,57 @@ struct ThreeP {
     static constexpr W24 V = make();
 };
 
-// A round's operands are requested while the one before is multiplied.  Two
-// column groups share the matrices' reads where every CU has a block of two
-// (2^15: 39 against 40 us) and then take a wavefront's whole register file.
-// The record is loaded late: requested before the last round it cost the
-// second wavefront per SIMD (2^15 in one group a block: 51 us).
-template <class F, int LOG_R, int G, bool LAST>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 1 ? 2 : 1))) void dense753_kernel(PassArgs<F> a)
+// A round's operands are requested while the one before is multiplied.  The
+// record is loaded late: requested before the last round it cost the second
+// wavefront per SIMD (2^15, KS = 4: 51 us).
+template <class F, int LOG_R, int KS, bool LAST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void dense753_kernel(PassArgs<F> a)
 {
-    using D = DenseWave<F, LOG_R, G>;
+    using D = DenseWave<F, LOG_R, KS>;
     constexpr uint32_t R = D::R;
-    __shared__ uint4 part[G * 3 * 6 * 64];
+    constexpr int G = 4 / KS;
+    static_assert(R / 2 / KS <= 32, "terms within DENSE_BIAS");
+    __shared__ uint4 part[G * (KS - 1) * 6 * 64];
     const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
     const uint32_t k = tile & (R / 2 - 1);
-    const int lane = (int)__lane_id(), wave = (int)uniform(threadIdx.x >> 6);
-    const size_t col = (size_t)(tile >> (LOG_R - 1)) * (32 * G) + (lane & 31);
+    const int lane = (int)__lane_id(), wave = (int)uniform(threadIdx.x >> 6), g = wave / KS, me = wave % KS;
+    const size_t col = ((size_t)(tile >> (LOG_R - 1)) * G + g) * 32 + (lane & 31);
 
-    v16i se[G][3], so[G][3];
+    v16i se[3], so[3];
 #pragma unroll
-    for (int g = 0; g < G; ++g)
+    for (int I = 0; I < 3; ++I)
 #pragma unroll
-        for (int I = 0; I < 3; ++I)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                se[g][I][i] = DENSE_BIAS;
-                so[g][I][i] = 0;
-            }
+        for (int i = 0; i < 16; ++i) {
+            se[I][i] = DENSE_BIAS;
+            so[I][i] = 0;
+        }
     typename D::Terms t;
-    D::load(t, a, k, col, 2 * wave);
+    D::load(t, a, k, col, 2 * me);
 #pragma unroll
     for (int r = 0; r + 1 < D::ROUNDS; ++r) {
         typename D::Terms next;
-        D::load(next, a, k, col, 8 * (r + 1) + 2 * wave);
+        D::load(next, a, k, col, 2 * (KS * (r + 1) + me));
         D::add(se, so, t, k & 1);
         __builtin_amdgcn_sched_barrier(0);
         t = next;
     }
     D::add(se, so, t, k & 1);
-    E753 y;
+    E753 y = D::finish(se, so);
+    uint4 *const p = part + g * (KS - 1) * 6 * 64 + lane;
+    if (me) {
 #pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const E753 v = D::finish(se[g], so[g]);
-        if (wave == g) {
-            y = v;
-        } else {
-            const int slot = (g * 3 + wave - (wave > g ? 1 : 0)) * 6;
-#pragma unroll
-            for (int q = 0; q < 6; ++q)
-                part[(slot + q) * 64 + lane] = make_uint4(v.v[4 * q], v.v[4 * q + 1], v.v[4 * q + 2], v.v[4 * q + 3]);
-        }
+        for (int q = 0; q < 6; ++q)
+            p[((me - 1) * 6 + q) * 64] = make_uint4(y.v[4 * q], y.v[4 * q + 1], y.v[4 * q + 2], y.v[4 * q + 3]);
     }
     __syncthreads();
-    if (wave >= G)  // wavefront g < G ends column group g
+    if (me)
         return;
 #pragma unroll
-    for (int p = 0; p < 3; ++p) {
+    for (int i = 0; i + 1 < KS; ++i) {
         unsigned c = 0;
 #pragma unroll
         for (int q = 0; q < 6; ++q) {
-            const uint4 v = part[((wave * 3 + p) * 6 + q) * 64 + lane];
+            const uint4 v = p[(i * 6 + q) * 64];
             y.v[4 * q] = __builtin_addc(y.v[4 * q], v.x, c, &c);
             y.v[4 * q + 1] = __builtin_addc(y.v[4 * q + 1], v.y, c, &c);
             y.v[4 * q + 2] = __builtin_addc(y.v[4 * q + 2], v.z, c, &c);
@@ -218,8 +205,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(G == 1 ? 2 
     }
     // where this lane's output goes, and its twiddle in the next pass
     const uint32_t kk = k + (lane >> 5) * (R / 2);
-    const size_t ns = (size_t)1 << a.log_ns, mine = col + 32 * (wave & (G - 1));
-    const size_t at = ((mine >> a.log_ns) << (a.log_ns + LOG_R)) + ((size_t)kk << a.log_ns) + (mine & (ns - 1));
+    const size_t ns = (size_t)1 << a.log_ns;
+    const size_t at = ((col >> a.log_ns) << (a.log_ns + LOG_R)) + ((size_t)kk << a.log_ns) + (col & (ns - 1));
     unsigned c = 0;
 #pragma unroll
     for (int i = 0; i < 24; ++i)
@@ -260,14 +247,14 @@ __global__ __launch_bounds__(64) void build_dense753_records_kernel(TW753 *out, 
     out[i] = F::make_tw(v);
 }
 
-template <class F, int LOG_R, int G>
+template <class F, int LOG_R, int KS>
 static void launch_r(const PassJob<F> &job, bool last, hipStream_t st)
 {
-    const dim3 grid((1u << (job.a.log_n - 6)) / G), block(256);
+    const dim3 grid((1u << (job.a.log_n - 8)) * KS), block(256);
     if (last)
-        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, G, true>), grid, block, 0, st, job.a);
+        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, true>), grid, block, 0, st, job.a);
     else
-        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, G, false>), grid, block, 0, st, job.a);
+        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, false>), grid, block, 0, st, job.a);
 }
 template <class F>
 void launch_dense753(const PassJob<F> &job, bool last, hipStream_t st)
@@ -277,9 +264,9 @@ void launch_dense753(const PassJob<F> &job, bool last, hipStream_t st)
         return;
     }
     switch (job.log_r) {
-    case 4: launch_r<F, 4, 1>(job, last, st); break;
-    case 5: launch_r<F, 5, 1>(job, last, st); break;
-    case 6: launch_r<F, 6, 1>(job, last, st); break;
+    case 4: launch_r<F, 4, 4>(job, last, st); break;
+    case 5: launch_r<F, 5, 4>(job, last, st); break;
+    case 6: launch_r<F, 6, 4>(job, last, st); break;
     default: break;
     }
 }

@@ -120,8 +120,7 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
 // and which need 32 columns.  Against the vector kernels, with other radices
 // in brackets, time on one box: 2^10 16 / 35 us, 2^11 18 / 40, 2^12 20 / 41
 // (three passes 22), 2^13 23 / 44 (2^7 2^6 25), 2^14 26 / 48 (2^7 2^7 30),
-// 2^15 39 / 57 (one column group a block 40, the passes below 50), 2^16 73 /
-// 60.
+// 2^15 36 / 57 (the passes below 50), 2^16 60-64 / 60.
 //
 // Others: passes of matrix753_kernels.h.  Radices of 2^4 .. 2^6 in tiles of
 // 32 columns, the first and the last at least 2^5 (their columns are k1 and

@@ -156,19 +156,19 @@ def test_passes_match_dft(radices):
 
 @pytest.mark.parametrize("field", FIELDS)
 def test_dense_sums_and_bounds(field):
-    """dense753.hip: column sums of up to 8 terms from 2^17 255, 25 limbs, the
+    """dense753.hip: column sums of up to 32 terms from 2^18 255, 25 limbs, the
     quotient from the top two in single precision, four such parts plus 3 p."""
     p = g.MODULI[field]
-    bias, row0 = 255 << 17, 1 << 17
+    bias, row0 = 255 << 18, 1 << 18
     top = np.float32((p >> 736) + ((p >> 704) & 0xFFFFFFFF) / 2.0 ** 32)
     inv = np.float32(1.0 / float(top))
-    assert 8 * 96 * 2 ** 14 < bias and 2 * p < OFFSET and -2 * p > -OFFSET
+    assert 32 * 96 * 2 ** 14 < bias and 2 * p < OFFSET and -2 * p > -OFFSET
     rng = random.Random(field + 100)
     for case in range(8):
         parts, exact = [], 0
         for _ in range(4):
             sums, want = np.full(96, bias, dtype=np.int64), 0
-            for _ in range(8):
+            for _ in range(32):
                 w = rng.choice([0, 1, p - 1, p // 2, p // 2 + 1, rng.randrange(p)])
                 cols = columns(w, p)
                 y = rng.choice([0, 4 * p, -2 * p, 2 * p - 1, rng.randrange(-2 * p, 4 * p)])
