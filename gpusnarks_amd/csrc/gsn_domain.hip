@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "batch_impl.h"
+#include "dot753.h"
 #include "gpusnarks.h"
 #include "gsn_internal.h"
 #include "mixed753.h"
@@ -806,19 +807,33 @@ int create_ext_plan(PlanBase **out, unsigned log_n, const void *shift, int inver
     return GSN_OK;
 }
 
-template <class O>
+template <int FID, class E>
+void launch_dot(E *partial, const E *a, const E *b, size_t n, unsigned blocks, hipStream_t st)
+{
+    if constexpr (FID == GSN_FIELD_FP32) {
+        hipLaunchKernelGGL(dot_kernel<Ops32>, dim3(blocks), dim3(DOT_THREADS), 0, st, partial, a, b, n);
+    } else {
+        using H = typename FieldInfo<FID>::Host;
+        // 2^-768, whose Montgomery form is 1
+        static const TW753 r_inv = [] {
+            const uint32_t one[24] = {1};
+            return make_tw753<H, typename FieldInfo<FID>::Params>(H::from_raw(one));
+        }();
+        launch_dot753<typename FieldInfo<FID>::Dev>(partial, a, b, n, blocks, r_inv, st);
+    }
+}
+
+template <int FID>
 int dot_t(void *d_out, const void *d_a, const void *d_b, size_t n, hipStream_t st)
 {
-    using E = typename O::elem;
-    const unsigned blocks = (unsigned)std::min<size_t>(1024, (n + DOT_THREADS - 1) / DOT_THREADS);
+    using E = typename FieldInfo<FID>::Dev::elem_t;
+    const unsigned blocks = (unsigned)std::min<size_t>(FID == GSN_FIELD_FP32 ? 1024 : DOT753_BLOCKS, (n + DOT_THREADS - 1) / DOT_THREADS);
     // block sums in stream-ordered scratch: concurrent calls on different
     // streams get their own
     void *partial = nullptr;
     GSN_TRY(hip_status(hipMallocAsync(&partial, blocks * sizeof(E), st), "hipMallocAsync"));
-    hipLaunchKernelGGL(dot_kernel<O>, dim3(blocks), dim3(DOT_THREADS), 0, st, (E *)partial, (const E *)d_a,
-                       (const E *)d_b, n);
-    hipLaunchKernelGGL(dot_kernel<O>, dim3(1), dim3(DOT_THREADS), 0, st, (E *)d_out, (const E *)partial,
-                       (const E *)nullptr, (size_t)blocks);
+    launch_dot<FID>((E *)partial, (const E *)d_a, (const E *)d_b, n, blocks, st);
+    launch_dot<FID>((E *)d_out, (const E *)partial, (const E *)nullptr, (size_t)blocks, 1, st);
     const int rc = hip_status(hipGetLastError(), "inner product launch");
     const int rf = hip_status(hipFreeAsync(partial, st), "hipFreeAsync");
     return rc ? rc : rf;
@@ -880,9 +895,9 @@ int gsn_inner_product(int field, void *d_out, const void *d_a, const void *d_b, 
     GSN_TRY(ensure_device());
     hipStream_t st = (hipStream_t)stream;
     switch (field) {
-    case GSN_FIELD_FP32: return dot_t<Ops32>(d_out, d_a, d_b, n, st);
-    case GSN_FIELD_MNT4753_FR: return dot_t<Ops753<Mnt4753FrParams>>(d_out, d_a, d_b, n, st);
-    default: return dot_t<Ops753<Mnt6753FrParams>>(d_out, d_a, d_b, n, st);
+    case GSN_FIELD_FP32: return dot_t<GSN_FIELD_FP32>(d_out, d_a, d_b, n, st);
+    case GSN_FIELD_MNT4753_FR: return dot_t<GSN_FIELD_MNT4753_FR>(d_out, d_a, d_b, n, st);
+    default: return dot_t<GSN_FIELD_MNT6753_FR>(d_out, d_a, d_b, n, st);
     }
 }
 

@@ -264,6 +264,24 @@ def cheap_residues(field, n, seed):
     return x
 
 
+# one product a thread, two, and past the 8 that a thread adds up unreduced
+@pytest.mark.parametrize("field", [g.FIELD_MNT4753_FR, g.FIELD_MNT6753_FR])
+@pytest.mark.parametrize("n", [65536, 65537, 8 * 65536, 8 * 65536 + 65])
+def test_inner_product_unreduced_sums(field, n):
+    p, L = g.MODULI[field], g.NLIMBS[field]
+    a, b = cheap_residues(field, n, 0x1D1 + n), cheap_residues(field, n, 0x2E1 + n)
+    top = np.frombuffer((p - 1).to_bytes(4 * L, "little"), dtype=np.uint32)
+    a[::2], b[::2] = top, top  # every other thread's sums are the largest there are
+    say("inner product field", field, "n", n)
+    da, db, dout = g.DeviceArray.from_numpy(a), g.DeviceArray.from_numpy(b), g.DeviceArray(4 * L)
+    g.inner_product(field, dout.ptr, da.ptr, db.ptr, n)
+    g.synchronize()
+    ra, rb = a.tobytes(), b.tobytes()
+    want = sum(int.from_bytes(ra[i:i + 4 * L], "little") * int.from_bytes(rb[i:i + 4 * L], "little")
+               for i in range(0, len(ra), 4 * L)) * pow(1 << (32 * L), -1, p) % p
+    assert int.from_bytes(dout.download((1, L)).tobytes(), "little") == want
+
+
 def mixed_roots(field, n1, a):
     from tests.oracle_lib import odd_root
     M, w = odd_root(field)
