@@ -32,6 +32,7 @@
 #include <vector>
 
 #include "batch_impl.h"
+#include "columns753.h"
 #include "dot753.h"
 #include "gpusnarks.h"
 #include "gsn_internal.h"
@@ -629,6 +630,53 @@ struct MixedPlan : PlanBase {
     // are columns of one group; below, lanes would need matrices of their
     // own.  525 x 2^12: 1.51 ms, with the vector passes 2.39 ms.
     bool matrix() const { return FID != GSN_FIELD_FP32 && a >= 6; }
+    // The radix-2 part as transforms of columns, after the transpose.
+    bool columns() const
+    {
+        uint32_t r1 = 0, r2 = 0;
+        return matrix() && columns_split(a, r1, r2);
+    }
+    DeviceBuffer fold1, fold2;
+    // byte matrices of the powers of wr, of order 2^a, for both passes
+    int build_columns(const H &wr)
+    {
+        if constexpr (FID != GSN_FIELD_FP32) {
+            using F = typename FieldInfo<FID>::Dev;
+            const uint32_t hb = (a + 1) / 2;
+            std::vector<TW> vlo((size_t)1 << hb);
+            std::vector<E753> vhi((size_t)1 << (a - hb));
+            H acc = H::one();
+            for (TW &t : vlo) {
+                t = record<FID>(acc);
+                acc = acc * wr;
+            }
+            const H step = acc;
+            acc = H::one();
+            for (E753 &v : vhi) {
+                acc.to_canonical(v.v);
+                acc = acc * step;
+            }
+            DeviceBuffer dlo, dhi;
+            GSN_TRY(dlo.alloc(vlo.size() * sizeof(TW)));
+            GSN_TRY(dhi.alloc(vhi.size() * sizeof(E753)));
+            GSN_TRY(hip_status(hipMemcpy(dlo.ptr, vlo.data(), vlo.size() * sizeof(TW), hipMemcpyHostToDevice),
+                               "hipMemcpy"));
+            GSN_TRY(hip_status(hipMemcpy(dhi.ptr, vhi.data(), vhi.size() * sizeof(E753), hipMemcpyHostToDevice),
+                               "hipMemcpy"));
+            uint32_t r1 = 0, r2 = 0;
+            columns_split(a, r1, r2);
+            const uint32_t e1 = (1u << r1) - 1u, e2 = ((1u << r2) - 1u) << r1;
+            GSN_TRY(fold1.alloc((size_t)e1 * MAT_BYTES));
+            GSN_TRY(fold2.alloc((size_t)e2 * MAT_BYTES));
+            launch_build_mat753<F>((uint4 *)fold1.ptr, e1, true, (const E753 *)dhi.ptr, (const TW753 *)dlo.ptr, hb, a,
+                                   0, 0, 0, false, nullptr, 0);
+            launch_build_mat753<F>((uint4 *)fold2.ptr, e2, true, (const E753 *)dhi.ptr, (const TW753 *)dlo.ptr, hb, a,
+                                   r1, 0, 0, false, nullptr, 0);
+            GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+            GSN_TRY(hip_status(hipStreamSynchronize(nullptr), "matrix tables"));
+        }
+        return GSN_OK;
+    }
 
     int init(uint32_t n1_, uint32_t a_, int inv)
     {
@@ -665,7 +713,8 @@ struct MixedPlan : PlanBase {
                 put(cs, mix_cs_offset(q) + q + e, (up - un) * half);
             }
         }
-        // base^e = lo[e mod 2^h] hi[e >> h] (hi scaled by n1^-1 for the inverse)
+        // base^e = lo[e mod 2^h] hi[e >> h] (hi scaled by n1^-1 for the
+        // inverse, by n^-1 if the rows do not carry n2^-1)
         while (((size_t)1 << (2 * h)) < n)
             ++h;
         const size_t nlo = (size_t)1 << h, nhi = (n + nlo - 1) >> h;
@@ -673,7 +722,7 @@ struct MixedPlan : PlanBase {
         acc = H::one();
         for (size_t e = 0; e < nlo; ++e, acc = acc * base)
             put(vlo, e, acc);
-        H hacc = inv ? H(n1).mul_inv() : H::one();
+        H hacc = inv ? H(columns() ? (uint32_t)n : n1).mul_inv() : H::one();
         for (size_t y = 0; y < nhi; ++y, hacc = hacc * acc)
             put(vhi, y, hacc);
         GSN_TRY(T.alloc(n1 * sizeof(TW)));
@@ -708,7 +757,11 @@ struct MixedPlan : PlanBase {
         }
         num_passes = 2;
         device_bytes = mat.bytes + (n1 + nlo + nhi + MIX_CS_ELEMS) * sizeof(TW) + (rad.count > 1 ? 2 : 1) * n * sizeof(E);
-        if (a > 0) {
+        if (columns()) {
+            GSN_TRY(build_columns(base.pow(n1)));
+            device_bytes += fold1.bytes + fold2.bytes;
+            num_passes += 2;
+        } else if (a > 0) {
             // the rows: radix-2 transforms over w^n1 (a primitive 2^a-th root)
             const H wr = w.pow(n1);
             std::vector<gsn_batch_item> items(n1);
@@ -740,7 +793,7 @@ struct MixedPlan : PlanBase {
                 if (matrix()) {
                     const MixedPass p{dst, src, n1, a, L, mat.ptr, (const char *)mat.ptr + (size_t)n1 * MAT_BYTES,
                                       (const TW753 *)lo.ptr, (const TW753 *)hi.ptr, h};
-                    launch_mixed_mat<typename FieldInfo<FID>::Dev>(p, q, last, st);
+                    launch_mixed_mat<typename FieldInfo<FID>::Dev>(p, q, last && !columns(), st);
                     src = dst;
                     L *= q;
                     continue;
@@ -759,6 +812,18 @@ struct MixedPlan : PlanBase {
             L *= q;
         }
         GSN_TRY(hip_status(hipGetLastError(), "mixed-radix launch"));
+        if constexpr (FID != GSN_FIELD_FP32) {
+            if (columns()) {
+                // the twiddles and the transpose into the caller's buffer,
+                // which the two passes leave and reach again
+                const MixedPass p{(E *)out, (const E *)ws.ptr, n1, a, n1, nullptr, nullptr,
+                                  (const TW753 *)lo.ptr, (const TW753 *)hi.ptr, h};
+                launch_mixed_twist<typename FieldInfo<FID>::Dev>(p, st);
+                launch_columns753<typename FieldInfo<FID>::Dev>((const E753 *)out, (E753 *)out, (E753 *)ws.ptr, a, n1,
+                                                                fold1.ptr, fold2.ptr, st);
+                return hip_status(hipGetLastError(), "mixed-radix columns launch");
+            }
+        }
         if (rows)
             GSN_TRY(rows->enqueue(st));
         hipLaunchKernelGGL(mixed_transpose_kernel<O>, dim3(blocks_for(n)), dim3(256), 0, st, (E *)out,

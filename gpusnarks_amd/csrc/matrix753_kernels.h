@@ -281,6 +281,12 @@ __device__ __forceinline__ void mat753_mul(const v4i (&b0)[3], const v4i (&b1)[3
 // The columns of the last pass are W consecutive k1.  n^-1 rides on the
 // column factors of the first MAT_MID pass.
 
+// Transforms of the columns of an array, lanes on adjacent ones
+// (columns753.hip): COL_FIRST is MAT_FIRST with the columns after the digits
+// j2 .., COL_LAST the second and last pass, k1 fixed and folded.  Their tiles
+// may end early.
+enum : int { COL_FIRST = 16, COL_LAST = 17 };
+
 // What a pass needs, held in scalar registers: jobs come through a table
 // whose loads the compiler takes for lane-varying.
 struct MatArgs {
@@ -288,6 +294,7 @@ struct MatArgs {
     void *out;
     const void *fold, *col, *fix;  // matrices: folded, per column, and the pair (1, 3) (null: none)
     uint32_t log_n, log_s, log_g, log_np, log_n1, flags, blk;
+    uint32_t cols;  // COL_FIRST, COL_LAST
 };
 __device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 template <class T>
@@ -304,7 +311,8 @@ __device__ __forceinline__ MatArgs mat_args(const PassJob<F> &j, uint32_t tile)
                    uniform((const void *)j.a.tw_pass_a), uniform(j.a.log_n),
                    uniform(j.a.log_s),                   uniform(j.a.log_g),
                    uniform(j.a.log_np),                  uniform(j.a.log_n1),
-                   uniform(j.a.flags),                   uniform(tile - j.first_tile)};
+                   uniform(j.a.flags),                   uniform(tile - j.first_tile),
+                   0u};
 }
 
 // LDS of a tile.  Exchanges pass three of a thread's four elements.  Where rows
@@ -330,7 +338,9 @@ struct MatTile {
     static constexpr int R = 1 << LOG_R, W = 1 << LOG_W, T = R * W / 4, UB = LOG_R - 2;
     static constexpr int LOG_CB = mat_log_cb(LOG_R), CB = 1 << LOG_CB, RS = CB + 1, PL = mat_plane(R * RS),
                          PH = mat_plane(R / 2 * (W + 1));
-    static constexpr bool FIRST = KIND == MAT_FIRST, MID = KIND == MAT_MID || KIND == MAT_MID2, LAST = KIND == MAT_LAST;
+    static constexpr bool FIRST = KIND == MAT_FIRST || KIND == COL_FIRST, MID = KIND == MAT_MID || KIND == MAT_MID2,
+                          LAST = KIND == MAT_LAST, ENDS = LAST || KIND == COL_LAST,
+                          COL = KIND == COL_FIRST || KIND == COL_LAST;
     typedef __attribute__((address_space(1))) const u32x4 gcq4;
     typedef __attribute__((address_space(1))) u32x4 gq4;
 
@@ -338,6 +348,7 @@ struct MatTile {
     uint4 *lds;
     const int t, c, u;
     uint32_t jj;
+    uint32_t valid = W;     // columns of the tile
     uint32_t kap;           // the folded digit, k(i-1)
     uint32_t top = 0;       // MAT_MID: jP of column 0
     uint32_t next = 0;      // MAT_MID: the digits between ji and jP
@@ -353,7 +364,18 @@ struct MatTile {
         if constexpr (FIRST) {
             kap = 0;
             in0 = out0 = (size_t)a.blk * W;
-            in_stride = out_stride = (size_t)1 << (a.log_n - LOG_R);
+            in_stride = out_stride = (size_t)(KIND == COL_FIRST ? a.cols : 1u) << (a.log_n - LOG_R);
+            if constexpr (KIND == COL_FIRST)
+                valid = (uint32_t)(in_stride - in0 < (size_t)W ? in_stride - in0 : (size_t)W);
+        } else if constexpr (KIND == COL_LAST) {
+            const uint32_t tiles = (a.cols + W - 1) / W;
+            kap = a.blk / tiles;
+            const uint32_t c0 = (a.blk - kap * tiles) * W;
+            valid = a.cols - c0 < (uint32_t)W ? a.cols - c0 : (uint32_t)W;
+            in0 = ((size_t)kap << LOG_R) * a.cols + c0;
+            in_stride = a.cols;
+            out0 = (size_t)kap * a.cols + c0;
+            out_stride = (size_t)a.cols << a.log_g;
         } else if constexpr (MID) {
             // tiles with the same k(i-1), which read the same matrices, are
             // neighbours
@@ -437,7 +459,7 @@ struct MatTile {
     }
     // the steps that reduce x0 first: inputs are below 2 B in MAT_MID, below
     // B in MAT_LAST and below 6 p after the two plain steps of MAT_FIRST
-    static constexpr bool reduces(int s) { return MID ? s % 2 == 0 : LAST ? s % 2 == 1 : s % 2 == 1 && s >= 3; }
+    static constexpr bool reduces(int s) { return MID ? s % 2 == 0 : ENDS ? s % 2 == 1 : s % 2 == 1 && s >= 3; }
 
     // step s on elements lo (bit clear) and up; kk = low K bits of jj plus
     // `more`: matrix entry ((2^s - 1) << log_g) + (kap << s) + kk
@@ -612,6 +634,8 @@ struct MatTile {
         }
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
+            if (COL && z[k] >= 6 * (int)valid)
+                continue;
             gq4 *p = o + (6 * out_stride * r[k] + z[k]);
 #pragma unroll
             for (int i = 0; i < N; ++i) {
@@ -684,7 +708,7 @@ struct MatTile {
         } else {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                x[e] = gload(in0 + in_row(e) * in_stride + c);
+                x[e] = gload(in0 + in_row(e) * in_stride + (COL ? min(c, (int)valid - 1) : c));
         }
         set_bias();
         if constexpr (FIRST) {
@@ -716,7 +740,7 @@ struct MatTile {
             step<1, 0>(x[1], x[3], 1u);
         }
         pairs<1>();
-        if constexpr (LAST) {
+        if constexpr (ENDS) {
 #pragma unroll
             for (int e = 0; e < 4; ++e)
                 x[e] = F::canon(M::from_offset(x[e]));

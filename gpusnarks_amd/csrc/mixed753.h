@@ -24,6 +24,10 @@ struct MixedPass {
 // 2^log_n2 >= 64 columns
 template <class F>
 void launch_mixed_mat(const MixedPass &a, uint32_t q, bool last, hipStream_t stream);
+// Instead of `last`: the product by w^(j2 k1) and the transpose, row j2 of n1
+// positions.
+template <class F>
+void launch_mixed_twist(const MixedPass &a, hipStream_t stream);
 // The matrices of `count` canonical residues.
 template <class F>
 void launch_build_mat753_values(uint4 *out, uint32_t count, const E753 *values, hipStream_t stream);

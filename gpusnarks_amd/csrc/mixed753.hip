@@ -141,6 +141,19 @@ __device__ __forceinline__ E753 mat753_sum(const v4i (*b0)[3], const v4i (*b1)[3
     return y;
 }
 
+// v w^e, canonical
+template <class F>
+__device__ __forceinline__ E753 twist(const E753 &v, const MixedPass &a, uint64_t e)
+{
+    E753 t;
+    unsigned c = 0;
+#pragma unroll
+    for (int l = 0; l < 24; ++l)
+        t.v[l] = __builtin_addc(v.v[l], MultipleOfP<typename F::params, 32>::V.v[l], c, &c);
+    t = F::mul(t, F::load_tw(a.lo, (size_t)(e & ((1ull << a.h) - 1))));
+    return F::canon(F::mul(t, F::load_tw(a.hi, (size_t)(e >> a.h))));
+}
+
 // One pass.  START: the first one (no twiddles, canonical inputs); LAST: also
 // times w^(j2 k1), canonical outputs.
 template <class F, int Q, bool START, bool LAST>
@@ -192,14 +205,7 @@ __device__ __forceinline__ void mixed_mat_body(const MixedPass &a)
         const uint32_t pos = pos0 + s * a.L;
         const size_t i = ((size_t)pos << a.log_n2) + j2;
         if constexpr (LAST) {
-            const uint64_t e = (uint64_t)j2 * pos;
-            E753 t;
-            unsigned c = 0;
-#pragma unroll
-            for (int l = 0; l < 24; ++l)
-                t.v[l] = __builtin_addc(v.v[l], MultipleOfP<P, 32>::V.v[l], c, &c);
-            t = F::mul(t, F::load_tw(a.lo, (size_t)(e & ((1ull << a.h) - 1))));
-            F::store(a.dst, i, F::canon(F::mul(t, F::load_tw(a.hi, (size_t)(e >> a.h)))));
+            F::store(a.dst, i, twist<F>(v, a, (uint64_t)j2 * pos));
         } else {
             F::store(a.dst, i, v);
         }
@@ -252,6 +258,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Q > 3 ? 1 :
     mixed_mat_body<F, Q, START, LAST>(a);
 }
 
+// dst[j2 n1 + pos] = src[pos n2 + j2] w^(j2 pos).  A block takes 64 rows j2 of
+// four neighbouring pos, so that their stores meet in the cache.  Products by
+// records bound it, which the transpose alone leaves the time for: at
+// 525 x 2^12 a transpose takes 107 us, the products in the last odd pass
+// 150 more there.
+template <class F>
+__global__ __launch_bounds__(256) void mixed_twist_kernel(MixedPass a)
+{
+    const uint32_t groups = (a.n1 + 3) / 4, g = blockIdx.x / groups;
+    const uint32_t pos = 4 * (blockIdx.x - g * groups) + (threadIdx.x >> 6);
+    const size_t j2 = (size_t)g * 64 + (threadIdx.x & 63);
+    if (pos < a.n1)
+        F::store(a.dst, j2 * a.n1 + pos,
+                 twist<F>(F::load(a.src, ((size_t)pos << a.log_n2) + j2), a, (uint64_t)j2 * pos));
+}
+
 // matrices of given residues, a block each
 template <class F>
 __global__ __launch_bounds__(128) void build_mat753_values_kernel(uint4 *out, const E753 *values)
@@ -288,6 +310,11 @@ void launch_mixed_mat(const MixedPass &a, uint32_t q, bool last, hipStream_t st)
     }
 }
 template <class F>
+void launch_mixed_twist(const MixedPass &a, hipStream_t st)
+{
+    hipLaunchKernelGGL(mixed_twist_kernel<F>, dim3(((a.n1 + 3) / 4) << (a.log_n2 - 6)), dim3(256), 0, st, a);
+}
+template <class F>
 void launch_build_mat753_values(uint4 *out, uint32_t count, const E753 *values, hipStream_t st)
 {
     hipLaunchKernelGGL(build_mat753_values_kernel<F>, dim3(count), dim3(128), 0, st, out, values);
@@ -295,6 +322,8 @@ void launch_build_mat753_values(uint4 *out, uint32_t count, const E753 *values, 
 
 template void launch_mixed_mat<FMnt4>(const MixedPass &, uint32_t, bool, hipStream_t);
 template void launch_mixed_mat<FMnt6>(const MixedPass &, uint32_t, bool, hipStream_t);
+template void launch_mixed_twist<FMnt4>(const MixedPass &, hipStream_t);
+template void launch_mixed_twist<FMnt6>(const MixedPass &, hipStream_t);
 template void launch_build_mat753_values<FMnt4>(uint4 *, uint32_t, const E753 *, hipStream_t);
 template void launch_build_mat753_values<FMnt6>(uint4 *, uint32_t, const E753 *, hipStream_t);
 
