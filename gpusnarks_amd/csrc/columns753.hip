@@ -1,7 +1,10 @@
 // Radix-2 transforms of the columns of an array, lanes on adjacent columns:
 // the passes of matrix753_kernels.h where every twiddle is the same for all
 // columns, so there are no column factors and the first pass has only
-// 2^r1 - 1 matrices.
+// 2^r1 - 1 matrices.  525 columns of 2^12 points, 206 MB: 159 and 194 us (2.6
+// and 2.1 TB/s; the second pass reads 2^r1 times as many matrices, and its
+// tiles of 525 columns are 3% empty), against 2 x 316 us for the vector
+// kernels on rows and 107 for the transpose after them.
 #include "columns753.h"
 
 #include "matrix753_kernels.h"

@@ -219,6 +219,8 @@ __global__ __launch_bounds__(256) void ext_inv_kernel(typename F::elem_t *a, con
 //   Y[k1][j2] = w^(j2 k1) sum_j1 x[n2 j1 + j2] w^(n2 j1 k1)   (mixed_pass_kernel)
 //   Z[k1][k2] = sum_j2 Y[k1][j2] w^(n1 j2 k2)                  (radix-2 plans on rows)
 //   X[k1 + n1 k2] = Z[k1][k2]                                   (mixed_transpose_kernel)
+// or, 753-bit with 2^8 <= n2 <= 2^12, the product by w^(j2 k1) and the
+// transpose second and the transforms of columns last (MixedPlan::columns).
 // The odd DFT of every column runs as radix-3/5/7 Stockham passes, one
 // kernel per pass over all columns (thread = column j2 x group j, adjacent
 // threads on adjacent columns, so every access is coalesced): a pass of
@@ -628,9 +630,13 @@ struct MixedPlan : PlanBase {
     static void put(std::vector<TW> &v, size_t i, const H &x) { v[i] = record<FID>(x); }
     // The odd passes run on the matrix cores wherever a wavefront's 64 lanes
     // are columns of one group; below, lanes would need matrices of their
-    // own.  525 x 2^12: 1.51 ms, with the vector passes 2.39 ms.
+    // own.  525 x 2^12, rows as a batch: 1.51 ms, with the vector passes 2.39.
     bool matrix() const { return FID != GSN_FIELD_FP32 && a >= 6; }
-    // The radix-2 part as transforms of columns, after the transpose.
+    // The radix-2 part as transforms of columns, after the transpose instead
+    // of before it, for the a that split into two passes (2^8 .. 2^12): 525 x
+    // 2^12 1.18 ms against 1.51 with the rows as a batch, 7 x 2^12 81 us
+    // against 119, and 3 x 2^8 37 against 62, where a wavefront is mostly
+    // clipped.
     bool columns() const
     {
         uint32_t r1 = 0, r2 = 0;

@@ -12,10 +12,12 @@
 // (13.8k matrix-core cycles) and about 3.3k vector instructions, against 24
 // products of about 1700 vector instructions in the vector kernel.  At
 // 525 x 2^12 (2.15 million elements, 413 MB read and written a pass) the
-// radix-7, 5, 5 passes take 156, 167 and 167 us (2.6 TB/s) against the vector
-// kernel's 504, 413 and 413, and the last, radix-3 one 317 against 401: its
-// two products by w^(j2 k1), which no two lanes share, stay vector ones.  The
-// others wait on memory with one or two wavefronts per SIMD.
+// radix-7, 5, 5, 3 passes take 156, 167, 167 and 112 us (2.6 to 3.7 TB/s)
+// against the vector kernel's 504, 413, 413 and 401, of which about 150 are
+// the two products by w^(j2 k1).  No two lanes share these, so they stay
+// vector ones: in the last pass (317 us) or, where a transpose follows, in
+// mixed_twist_kernel.  The others wait on memory with one or two wavefronts
+// per SIMD.
 //
 // Values between the passes are small signed numbers, in two's complement
 // modulo 2^768.  Bounds: inputs of the first pass are below p, every further
@@ -259,10 +261,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Q > 3 ? 1 :
 }
 
 // dst[j2 n1 + pos] = src[pos n2 + j2] w^(j2 pos).  A block takes 64 rows j2 of
-// four neighbouring pos, so that their stores meet in the cache.  Products by
-// records bound it, which the transpose alone leaves the time for: at
-// 525 x 2^12 a transpose takes 107 us, the products in the last odd pass
-// 150 more there.
+// four neighbouring pos, so that their stores meet in the cache.  The products
+// by records bound it, with the transpose under them: 258 us at 525 x 2^12,
+// where a transpose alone takes 107 and the products cost the last odd pass
+// 205.
 template <class F>
 __global__ __launch_bounds__(256) void mixed_twist_kernel(MixedPass a)
 {

@@ -313,13 +313,18 @@ def test_mixed_radix_matches_oracle(orc, field, n1, a):
     assert np.array_equal(e.download(x.shape), x)
 
 
-# The odd passes' 64-column wavefronts start at a = 6: both sides of it, each
-# radix as the only, the first, a middle and the last pass.
+# The odd passes' 64-column wavefronts start at a = 6, and the radix-2 part
+# goes by columns from a = 8 to 12: both sides of these, each radix as the
+# only, the first, a middle and the last pass, and fewer and more columns than
+# a tile has.
 @pytest.mark.parametrize("field,n1,a", [(g.FIELD_MNT4753_FR, 3, 6), (g.FIELD_MNT4753_FR, 5, 7),
                                         (g.FIELD_MNT4753_FR, 7, 6), (g.FIELD_MNT4753_FR, 21, 5),
                                         (g.FIELD_MNT4753_FR, 25, 6), (g.FIELD_MNT6753_FR, 35, 6),
                                         (g.FIELD_MNT6753_FR, 49, 6), (g.FIELD_MNT6753_FR, 63, 6),
-                                        (g.FIELD_MNT6753_FR, 245, 8)])
+                                        (g.FIELD_MNT6753_FR, 245, 8), (g.FIELD_MNT4753_FR, 3, 8),
+                                        (g.FIELD_MNT4753_FR, 35, 8), (g.FIELD_MNT6753_FR, 15, 7),
+                                        (g.FIELD_MNT4753_FR, 5, 10), (g.FIELD_MNT6753_FR, 21, 11),
+                                        (g.FIELD_MNT4753_FR, 7, 12), (g.FIELD_MNT4753_FR, 3, 13)])
 def test_mixed_radix_column_groups(orc, field, n1, a):
     n = n1 << a
     p, L = g.MODULI[field], g.NLIMBS[field]
