@@ -12,9 +12,10 @@ constexpr bool dense_supported(const PassCfg &c)
 }
 
 // A Stockham pass: tw_col holds the matrices of w_R^e (e < R), tw_pass the
-// records that outputs take along to the next pass, of radix 2^log_np.
+// records that outputs take along to the next pass, of radix 2^log_np.  Of
+// `count` transforms, one after the other in both buffers.
 template <class F>
-void launch_dense753(const PassJob<F> &job, bool last, hipStream_t stream);
+void launch_dense753(const PassJob<F> &job, bool last, uint32_t count, hipStream_t stream);
 // The tables of a pass of radix 2^log_r (mat, or null) and, with 2^log_s
 // points through it and the ones before and a next pass of 2^log_next, its
 // records w_n^(j c n / 2^(log_s + log_next)) at (j << log_s) + c (rec, or

@@ -155,6 +155,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
     using D = DenseWave<F, LOG_R, KS>;
     constexpr uint32_t R = D::R;
     constexpr int G = 4 / KS;
+    a.in += (size_t)blockIdx.y << a.log_n;
+    a.out += (size_t)blockIdx.y << a.log_n;
     static_assert(R / 2 / KS <= 32, "terms within DENSE_BIAS");
     __shared__ uint4 part[G * (KS - 1) * 6 * 64];
     const uint32_t tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -248,25 +250,25 @@ __global__ __launch_bounds__(64) void build_dense753_records_kernel(TW753 *out, 
 }
 
 template <class F, int LOG_R, int KS>
-static void launch_r(const PassJob<F> &job, bool last, hipStream_t st)
+static void launch_r(const PassJob<F> &job, bool last, uint32_t count, hipStream_t st)
 {
-    const dim3 grid((1u << (job.a.log_n - 8)) * KS), block(256);
+    const dim3 grid((1u << (job.a.log_n - 8)) * KS, count), block(256);
     if (last)
         hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, true>), grid, block, 0, st, job.a);
     else
         hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, false>), grid, block, 0, st, job.a);
 }
 template <class F>
-void launch_dense753(const PassJob<F> &job, bool last, hipStream_t st)
+void launch_dense753(const PassJob<F> &job, bool last, uint32_t count, hipStream_t st)
 {
     if (job.log_w == 6) {
-        launch_r<F, 5, 2>(job, last, st);
+        launch_r<F, 5, 2>(job, last, count, st);
         return;
     }
     switch (job.log_r) {
-    case 4: launch_r<F, 4, 4>(job, last, st); break;
-    case 5: launch_r<F, 5, 4>(job, last, st); break;
-    case 6: launch_r<F, 6, 4>(job, last, st); break;
+    case 4: launch_r<F, 4, 4>(job, last, count, st); break;
+    case 5: launch_r<F, 5, 4>(job, last, count, st); break;
+    case 6: launch_r<F, 6, 4>(job, last, count, st); break;
     default: break;
     }
 }
@@ -287,7 +289,7 @@ void launch_build_dense753(uint4 *mat, uint32_t log_r, TW753 *rec, uint32_t log_
 }
 
 #define GSN_DENSE_FIELD(F)                                                                                        \
-    template void launch_dense753<F>(const PassJob<F> &, bool, hipStream_t);                                      \
+    template void launch_dense753<F>(const PassJob<F> &, bool, uint32_t, hipStream_t);                                    \
     template void launch_build_dense753<F>(uint4 *, uint32_t, TW753 *, uint32_t, uint32_t, const E753 *,          \
                                            const TW753 *, uint32_t, uint32_t, const TW753 *, hipStream_t);
 GSN_DENSE_FIELD(FMnt4)

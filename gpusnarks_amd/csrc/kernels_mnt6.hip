@@ -36,7 +36,7 @@ void launch_pass<FMnt6>(const PassJob<FMnt6> &job, const PassCfg &c, hipStream_t
 {
     const size_t grid = ((size_t)1 << (job.a.log_n - c.log_r)) >> c.log_w;
     if (c.kind == MAT_DENSE)
-        launch_dense753<FMnt6>(job, (job.a.flags & PASS_CANON) != 0, st);
+        launch_dense753<FMnt6>(job, (job.a.flags & PASS_CANON) != 0, 1, st);
     else if (c.kind)
         launch_mat<FMnt6>(job, nullptr, nullptr, (uint32_t)grid, c, st);
     else

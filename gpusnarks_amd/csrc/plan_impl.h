@@ -7,6 +7,7 @@
 #include <cstring>
 #include <vector>
 
+#include "dense753.h"
 #include "device_field.h"
 #include "gpusnarks.h"
 #include "gsn_internal.h"
@@ -242,6 +243,24 @@ struct PlanImpl final : PlanBase {
         for (size_t i = 0; i < jobs.size(); ++i) {
             launch_pass<F>(jobs[i], cfg[i], s);
             GSN_TRY(hip_status(hipGetLastError(), "ntt pass launch"));
+        }
+        return GSN_OK;
+    }
+
+    // Two transforms next to each other in both buffers, in the same launches
+    // (dense passes only).
+    bool dense() const { return !cfg.empty() && cfg[0].kind == MAT_DENSE; }
+    int execute_two(const void *in, void *out, hipStream_t s)
+    {
+        if constexpr (!IS32) {
+            for (int i = 0; i < workspace_buffers; ++i)
+                GSN_TRY(scratch[i].alloc(((size_t)2 << log_n) * sizeof(elem)));
+            std::vector<PassJob<F>> jobs;
+            make_jobs(in, out, scratch[0].ptr, scratch[1].ptr, jobs);
+            for (size_t i = 0; i < jobs.size(); ++i) {
+                launch_dense753<F>(jobs[i], i + 1 == jobs.size(), 2, s);
+                GSN_TRY(hip_status(hipGetLastError(), "ntt pass launch"));
+            }
         }
         return GSN_OK;
     }

@@ -212,6 +212,25 @@ def test_extended_domain_matches_oracle(orc, field, log_n, custom_shift):
     assert np.array_equal(e.download(x.shape), x)
 
 
+# halves of 2^9 (a batch) and of every size that takes dense passes
+@pytest.mark.parametrize("field,log_n", [(g.FIELD_MNT4753_FR, l) for l in (10, 11, 12, 13, 14, 15)] +
+                         [(g.FIELD_MNT6753_FR, 16), (g.FIELD_MNT6753_FR, 17)])
+def test_extended_domain_dense_halves(orc, field, log_n):
+    x = cheap_residues(field, 1 << log_n, 0xED0 + log_n)
+    shift = mont(field, QNR[field])
+    say("extended domain halves field", field, "log_n", log_n)
+    want = orc.extended_fft(field, x, g.root_of_unity(field, log_n - 1), shift)
+    fwd, inv = g.Plan.extended(field, log_n), g.Plan.extended(field, log_n, inverse=True)
+    d, e = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+    for _ in range(2):
+        fwd.execute(d.ptr, e.ptr)
+        g.synchronize()
+        assert np.array_equal(e.download(x.shape), want)
+    inv.execute(e.ptr, e.ptr)  # in place
+    g.synchronize()
+    assert np.array_equal(e.download(x.shape), x)
+
+
 def test_extended_domain_errors():
     one = mont(g.FIELD_MNT6753_FR, 1)
     with pytest.raises(g.GsnError):
