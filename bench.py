@@ -4,8 +4,9 @@
 Headline: butterflies/s of a forward NTT over the 753-bit field MNT6-753 Fr
 at n = 2^18 (24 x u32 Montgomery limbs per element, operands resident in
 HBM), one transform per step.  The same line carries:
-  roofline      the pass kernel against the integer-multiply (v_mad_u64_u32)
-                peak, with its measured average launch time;
+  roofline      the transform against the integer-multiply (v_mad_u64_u32)
+                peak, its products counted at 1176 multiply-adds however they
+                are formed, with the measured average launch time of a pass;
   cpu_baseline  the oracle's restatement of the reference host FFT
                 (test/fft_host.h, log_cpus = 10 as test/main.cpp:71) on this
                 host's cores, on a bounded sample;
@@ -184,7 +185,7 @@ def bench_inner_product(log_n=18, reps=20):
     e1.synchronize()
     ms = g.Event.elapsed_ms(e0, e1) / reps
     return {"field": "MNT4-753 Fr", "n": a.shape[0], "ms": ms, "products_per_s": a.shape[0] / (ms * 1e-3),
-            "note": "general 753-bit Montgomery products (1431 multiply-adds each) plus a two-level sum"}
+            "note": "729 multiply-adds a product, summed unreduced in each thread, plus a two-level sum"}
 
 
 def cpu_info():
@@ -613,9 +614,10 @@ def main():
         "bound": "valu-int-mul", "unit": "Tmad/s",
         "achieved": achieved / 1e12, "peak": MAD_PEAK / 1e12, "frac": achieved / MAD_PEAK,
         "traffic": None,
-        "kernel": "ntt753_kernel (one Stockham pass, radix 2^%d)" % (log_n // passes),
+        "kernel": "mat753_kernel (one of %d passes; products as int8 MFMA, so the fraction of the vector "
+                  "multiply rate is a rate of equivalents, and no bound)" % passes,
         "launches_per_step": passes, "avg_launch_ms": ms_launch,
-        "work_per_launch": "%d butterflies x 1176 v_mad_u64_u32" % (bfly(log_n) // passes),
+        "work_per_launch": "%d butterflies x 1176 multiply-adds" % (bfly(log_n) // passes),
         "peak_note": "256 CU x 64 lanes/clk x 2.4 GHz (peak engine clock); clock_measured_ghz is the engine "
                      "clock while the 753-bit product runs on every CU (gsn_debug_clock_ghz)",
     }
