@@ -33,6 +33,7 @@
 
 #include "batch_impl.h"
 #include "columns753.h"
+#include "coset753.h"
 #include "dot753.h"
 #include "gpusnarks.h"
 #include "gsn_internal.h"
@@ -377,10 +378,51 @@ typename FieldInfo<FID>::Host value_r()
     return H::from_canonical(H::one().im_rep);  // one() holds R mod p
 }
 
+// the residue of a twiddle record
+inline void value_of(E753 &v, const TW753 &t)
+{
+    for (int l = 0; l < 24; ++l) {
+        uint64_t x = 0;
+        for (int d = 32 * l / 29; d < 26 && 29 * d < 32 * l + 32; ++d) {
+            const int at = 29 * d - 32 * l;
+            x |= at >= 0 ? (uint64_t)t.w[d] << at : (uint64_t)t.w[d] >> -at;
+        }
+        v.v[l] = (uint32_t)x;
+    }
+}
+
+// byte matrices of the residues of records
+template <int FID>
+int build_matrices(DeviceBuffer &mat, const std::vector<TW753> &records)
+{
+    std::vector<E753> vals(records.size());
+    for (size_t i = 0; i < vals.size(); ++i)
+        value_of(vals[i], records[i]);
+    DeviceBuffer dv;
+    GSN_TRY(dv.alloc(vals.size() * sizeof(E753)));
+    GSN_TRY(hip_status(hipMemcpy(dv.ptr, vals.data(), vals.size() * sizeof(E753), hipMemcpyHostToDevice), "hipMemcpy"));
+    GSN_TRY(mat.alloc(vals.size() * MAT_BYTES));
+    launch_build_mat753_values<typename FieldInfo<FID>::Dev>((uint4 *)mat.ptr, (uint32_t)vals.size(),
+                                                             (const E753 *)dv.ptr, 0);
+    GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+    return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
+}
+
 struct CosetTables {
     DeviceBuffer lo, hi;
+    DeviceBuffer mat;  // hi as byte matrices (coset_matrix)
     uint32_t h = 0;
+    CosetArgs args() const { return CosetArgs{(const TW753 *)lo.ptr, mat.ptr, h}; }
 };
+// Whether hi's products go to the matrix cores: 64 consecutive i share one
+// from 2^11 points (7.0 against 8.9 us there, 95 against 117 at 2^20).  These
+// tables outlive the calls, and at 9216 B a power (224 as a record) they would
+// pass 10 MB each beyond 2^20.
+template <int FID>
+constexpr bool coset_matrix(unsigned log_n)
+{
+    return FID != GSN_FIELD_FP32 && log_n >= 11 && log_n <= 20;
+}
 
 std::mutex g_coset_mutex;
 std::map<std::tuple<int, unsigned, int, std::vector<uint32_t>>, std::unique_ptr<CosetTables>> g_coset;
@@ -415,6 +457,9 @@ int coset_tables(CosetTables **out, const typename FieldInfo<FID>::Host &g, unsi
         GSN_TRY(t->hi.alloc(nhi * sizeof(tw)));
         GSN_TRY(hip_status(hipMemcpy(t->lo.ptr, lo.data(), nlo * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
         GSN_TRY(hip_status(hipMemcpy(t->hi.ptr, hi.data(), nhi * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
+        if constexpr (FID != GSN_FIELD_FP32)
+            if (coset_matrix<FID>(log_n))
+                GSN_TRY(build_matrices<FID>(t->mat, hi));
         slot = std::move(t);
     }
     *out = slot.get();
@@ -442,6 +487,12 @@ int coset_t(void *out, const void *in, size_t n, const void *g_limbs, int invers
         return set_error(GSN_ERR_INVALID_ARGUMENT, "the coset generator must be a nonzero canonical element");
     CosetTables *t = nullptr;
     GSN_TRY(coset_tables<FID>(&t, g, log_n, inverse));
+    if constexpr (FID != GSN_FIELD_FP32) {
+        if (coset_matrix<FID>(log_n)) {
+            launch_coset753<F>((E753 *)out, (const E753 *)in, t->args(), n, st);
+            return hip_status(hipGetLastError(), "coset launch");
+        }
+    }
     hipLaunchKernelGGL(ew_coset_kernel<F>, dim3(blocks_for(n)), dim3(256), 0, st, (typename F::elem_t *)out,
                        (const typename F::elem_t *)in, (const typename F::tw_t *)t->lo.ptr,
                        (const typename F::tw_t *)t->hi.ptr, t->h, n);
@@ -512,6 +563,7 @@ struct ExtPlan : PlanBase {
     PlanBase *half = nullptr;
     CosetTables *tab = nullptr;  // g^i (forward) or g^-i (inverse), i < m
     typename F::tw_t c;          // G (forward) or 1 / (1 - G) (inverse)
+    DeviceBuffer cmat;           // its matrix (coset_matrix)
     std::unique_ptr<BatchImpl> halves;  // both half transforms, fused
     const void *halves_in = nullptr;
     void *halves_out = nullptr;
@@ -520,7 +572,7 @@ struct ExtPlan : PlanBase {
     // both size-m transforms of in[0, m), in[m, 2m) into out[0, m), out[m, 2m)
     // A batch of two or, where one transform alone takes dense passes, both
     // in the same launches of these: 2^11 points in all 31 us, with the batch
-    // 52, 2^13 37 / 60, 2^15 55 / 69, 2^16 72 / 72.
+    // 52, 2^13 32 / 55, 2^15 50 / 65, 2^16 69 / 69.
     int run_halves(const void *in, void *out, hipStream_t st)
     {
         auto *h = static_cast<PlanImpl<FID> *>(half);
@@ -540,6 +592,18 @@ struct ExtPlan : PlanBase {
         return halves->enqueue(st);
     }
 
+    // the elementwise step with its shared factors on the matrix cores
+    bool matrix_step(const void *in, void *out, size_t m, hipStream_t st)
+    {
+        if constexpr (FID != GSN_FIELD_FP32) {
+            if (coset_matrix<FID>(log_n - 1)) {
+                launch_ext753<F>((E753 *)out, (const E753 *)in, tab->args(), cmat.ptr, m, inverse, st);
+                return true;
+            }
+        }
+        return false;
+    }
+
     int init(unsigned L, const H &g, int inv)
     {
         field = FID;
@@ -552,6 +616,9 @@ struct ExtPlan : PlanBase {
         GSN_TRY(create_plan(&half, FID, lm, nullptr, inv));
         GSN_TRY(coset_tables<FID>(&tab, g, lm, inv));
         c = inv ? record<FID>((H::one() - G).mul_inv()) : record<FID>(G);
+        if constexpr (FID != GSN_FIELD_FP32)
+            if (coset_matrix<FID>(lm))
+                GSN_TRY(build_matrices<FID>(cmat, {c}));
         num_passes = half->num_passes + 1;  // the halves' passes are fused
         device_bytes = half->device_bytes;
         return GSN_OK;
@@ -565,13 +632,16 @@ struct ExtPlan : PlanBase {
         const auto *lo = (const typename F::tw_t *)tab->lo.ptr, *hi = (const typename F::tw_t *)tab->hi.ptr;
         if (!inverse) {
             GSN_TRY(take_injected_fault());
-            hipLaunchKernelGGL(ext_fwd_kernel<F>, grid, block, 0, st, (E *)out, (const E *)in, lo, hi, tab->h, c, m);
+            if (!matrix_step(in, out, m, st))
+                hipLaunchKernelGGL(ext_fwd_kernel<F>, grid, block, 0, st, (E *)out, (const E *)in, lo, hi, tab->h, c,
+                                   m);
             GSN_TRY(hip_status(hipGetLastError(), "extended-domain launch"));
             return run_halves(out, out, st);
         }
         GSN_TRY(run_halves(in, out, st));
         GSN_TRY(take_injected_fault());
-        hipLaunchKernelGGL(ext_inv_kernel<F>, grid, block, 0, st, (E *)out, lo, hi, tab->h, c, m);
+        if (!matrix_step(out, out, m, st))
+            hipLaunchKernelGGL(ext_inv_kernel<F>, grid, block, 0, st, (E *)out, lo, hi, tab->h, c, m);
         return hip_status(hipGetLastError(), "extended-domain launch");
     }
 };
@@ -607,19 +677,6 @@ struct MixInfo<GSN_FIELD_MNT6753_FR> {
 // standard 2^a-th root times ROOT_ODD^(ODD_MAX / n1)): the odd-DFT kernel
 // into the plan's workspace, n1 radix-2 transforms of its rows as one
 // batch, and the transpose into the output.
-// the residue of a twiddle record
-inline void value_of(E753 &v, const TW753 &t)
-{
-    for (int l = 0; l < 24; ++l) {
-        uint64_t x = 0;
-        for (int d = 32 * l / 29; d < 26 && 29 * d < 32 * l + 32; ++d) {
-            const int at = 29 * d - 32 * l;
-            x |= at >= 0 ? (uint64_t)t.w[d] << at : (uint64_t)t.w[d] >> -at;
-        }
-        v.v[l] = (uint32_t)x;
-    }
-}
-
 template <int FID>
 struct MixedPlan : PlanBase {
     using H = typename FieldInfo<FID>::Host;
@@ -751,20 +808,9 @@ struct MixedPlan : PlanBase {
         GSN_TRY(hip_status(hipMemcpy(hi.ptr, vhi.data(), nhi * sizeof(TW), hipMemcpyHostToDevice), "hipMemcpy"));
         if constexpr (FID != GSN_FIELD_FP32) {
             if (matrix()) {
-                std::vector<E753> vals(n1 + MIX_CS_ELEMS);
-                for (uint32_t e = 0; e < n1; ++e)
-                    value_of(vals[e], t[e]);
-                for (uint32_t e = 0; e < MIX_CS_ELEMS; ++e)
-                    value_of(vals[n1 + e], cs[e]);
-                DeviceBuffer dv;
-                GSN_TRY(dv.alloc(vals.size() * sizeof(E753)));
-                GSN_TRY(hip_status(hipMemcpy(dv.ptr, vals.data(), vals.size() * sizeof(E753), hipMemcpyHostToDevice),
-                                   "hipMemcpy"));
-                GSN_TRY(mat.alloc(vals.size() * MAT_BYTES));
-                launch_build_mat753_values<typename FieldInfo<FID>::Dev>((uint4 *)mat.ptr, (uint32_t)vals.size(),
-                                                                         (const E753 *)dv.ptr, 0);
-                GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
-                GSN_TRY(hip_status(hipStreamSynchronize(nullptr), "matrix tables"));
+                std::vector<TW753> both(t.begin(), t.end());
+                both.insert(both.end(), cs.begin(), cs.end());
+                GSN_TRY(build_matrices<FID>(mat, both));
             }
         }
         num_passes = 2;

@@ -270,7 +270,10 @@ struct PlanImpl final : PlanBase {
     size_t workspace_bytes() const override
     {
         const size_t one = ((size_t)1 << log_n) * sizeof(elem);
-        const int nb = workspace_buffers;
+        // (Four matrix passes work in one buffer, but what the caller has to
+        // bring, and so which sizes a fixed workspace takes, stays what any
+        // other schedule of these sizes needs.)
+        const int nb = !IS32 && cfg.size() > 3 ? 2 : workspace_buffers;
         return nb == 0 ? 0 : nb == 1 ? one : ((one + 255) & ~(size_t)255) + one;
     }
 

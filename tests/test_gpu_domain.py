@@ -301,6 +301,32 @@ def test_inner_product_unreduced_sums(field, n):
     assert int.from_bytes(dout.download((1, L)).tobytes(), "little") == want
 
 
+# the matrices of hi's powers serve 2^11 to 2^20
+@pytest.mark.parametrize("field,log_n", [(f, l) for f in (g.FIELD_MNT4753_FR, g.FIELD_MNT6753_FR)
+                                         for l in (10, 11, 12)] + [(g.FIELD_MNT6753_FR, 20), (g.FIELD_MNT6753_FR, 21)])
+def test_coset_shift_shared_powers(field, log_n):
+    n, p, L = 1 << log_n, g.MODULI[field], g.NLIMBS[field]
+    x = cheap_residues(field, n, 0xC05 + log_n)
+    ends = [np.frombuffer(v.to_bytes(4 * L, "little"), dtype=np.uint32) for v in (p - 1, 0, 1)]
+    for i in range(0, n, 7):
+        x[i] = ends[i % 3]
+    gen = residues(field, 8, 0xC0 + field)[3]
+    say("coset shift field", field, "log_n", log_n)
+    r = pow(1 << (32 * L), -1, p)
+    gi = int.from_bytes(gen.tobytes(), "little") * r % p
+    d, e = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+    g.coset_shift(field, e.ptr, d.ptr, n, gen)
+    g.synchronize()
+    got = e.download(x.shape)
+    rows = range(n) if log_n <= 12 else [0, 1, 6, 7, 63, 64, n // 2 - 1, n // 2, n - 7, n - 1]
+    for i in rows:
+        want = int.from_bytes(x[i].tobytes(), "little") * pow(gi, i, p) % p
+        assert int.from_bytes(got[i].tobytes(), "little") == want, i
+    g.coset_shift(field, e.ptr, e.ptr, n, gen, inverse=True)  # in place
+    g.synchronize()
+    assert np.array_equal(e.download(x.shape), x)
+
+
 def mixed_roots(field, n1, a):
     from tests.oracle_lib import odd_root
     M, w = odd_root(field)
