@@ -55,6 +55,8 @@ struct BatchMemory {
     hipStream_t stream = nullptr;
 };
 
+// Which schedules the items of a batch take together.
+std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count);
 // Workspace bytes a batch of these items needs (256-byte aligned slices).
 size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count);
 // Builds the schedule.

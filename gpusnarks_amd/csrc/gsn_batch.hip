@@ -131,11 +131,46 @@ int BatchImpl::launch(hipStream_t s)
     return enqueue(s);
 }
 
+// Matrix passes of different sizes share a launch only where their radices
+// agree, and 2^15 points are 32 tiles of 2^10; the vector kernels' 2^15 .. 2^18
+// share all launches, at 50 us for every 256 tiles of 2^9.  So, in units of
+// 2^15 points, matrix against vector: 2^15 alone 55 / 63 us, but 2^16 74 / 69,
+// 2^17 85 / 76, 2^15 and 2^16 (3 units) 96 / 74; past four units 2 x 2^17
+// 97 / 128, 2^15 and 2 x 2^16 102 / 122, but with both 2^16 and 2^17, which
+// share next to nothing, 2^16 and 2^17 (6) 155 / 122, 2^15 .. 2^17 (7)
+// 157 / 123, and two of each with smaller ones (12) 239 / 228; two of each of
+// 2^15 .. 2^17 (14) 186 / 221, 2^16 .. 2^18 (14) 200 / 228.
+std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count)
+{
+    struct Load {
+        size_t units = 0;
+        bool above = false, has16 = false, has17 = false;
+        bool few() const { return units <= 4 ? above : units <= 12 && has16 && has17; }
+    } load[3];
+    for (size_t i = 0; i < count; ++i) {
+        const int f = items[i].field;
+        const unsigned L = items[i].log_n;
+        if ((f != GSN_FIELD_MNT4753_FR && f != GSN_FIELD_MNT6753_FR) || L < 15 || (int)L > two_adicity(f))
+            continue;
+        load[f].units += (size_t)1 << (L - 15);
+        load[f].above |= L > 15;
+        load[f].has16 |= L == 16;
+        load[f].has17 |= L == 17;
+    }
+    std::vector<PlanUse> uses(count, FUSED);
+    for (size_t i = 0; i < count; ++i)
+        if (items[i].log_n >= 15 && items[i].log_n <= 17 && items[i].field > 0 && items[i].field < 3 &&
+            load[items[i].field].few())
+            uses[i] = FUSED_FEW;
+    return uses;
+}
+
 size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count)
 {
+    const std::vector<PlanUse> uses = batch_uses(items, count);
     size_t bytes = 0;
     for (size_t i = 0; i < count; ++i) {
-        const std::vector<PassCfg> v = choose_passes(items[i].field, items[i].log_n, true);
+        const std::vector<PassCfg> v = choose_passes(items[i].field, items[i].log_n, uses[i]);
         const int nbuf = schedule_buffers(v);
         bytes += (size_t)nbuf * ((size_t)1 << items[i].log_n) * element_bytes(items[i].field);
         bytes = (bytes + 255) & ~(size_t)255;
@@ -148,13 +183,14 @@ int build_batch(BatchImpl &b, const gsn_batch_item *items, size_t count, int use
     GSN_TRY(ensure_device());
     // plans and workspace sizes
     std::vector<PlanBase *> plans(count);
+    const std::vector<PlanUse> uses = batch_uses(items, count);
     size_t ws_bytes = 0;
     std::vector<size_t> ws_off(count);
     for (size_t i = 0; i < count; ++i) {
         const gsn_batch_item &it = items[i];
         if (!it.d_in || !it.d_out)
             return set_error(GSN_ERR_INVALID_ARGUMENT, "batch item " + std::to_string(i) + " has a NULL buffer");
-        GSN_TRY(cached_plan(&plans[i], it.field, it.log_n, it.omega, it.inverse, true));
+        GSN_TRY(cached_plan(&plans[i], it.field, it.log_n, it.omega, it.inverse, uses[i]));
         const size_t eb = element_bytes(it.field);
         const size_t n = (size_t)1 << it.log_n;
         const int nbuf = plans[i]->workspace_buffers;

@@ -44,6 +44,11 @@ struct DeviceBuffer {
     int alloc(size_t n);  // grows; contents are not preserved
 };
 
+// How a plan's passes run, which its schedule depends on: by themselves, or
+// fused with other transforms' (the batch table's schedules), FUSED_FEW where
+// these are too few to fill the matrix passes (batch_uses).
+enum PlanUse : int { ALONE = 0, FUSED = 1, FUSED_FEW = 2 };
+
 // A transform plan: field, size, direction, twiddles and workspace.
 struct PlanBase {
     int field = 0;
@@ -51,7 +56,7 @@ struct PlanBase {
     int inverse = 0;
     int num_passes = 0;
     int workspace_buffers = 0;  // buffers of n elements an execution of a power-of-two plan needs
-    bool batch_mode = false;  // schedule of the batch table (fused launches)
+    PlanUse use = ALONE;
     size_t device_bytes = 0;
     std::mutex host_mutex;  // serialises the host entry point's buffer
     DeviceBuffer host_buf;
@@ -76,12 +81,10 @@ struct PlanBase {
 int staged_h2d(void *dev, const void *host, size_t bytes, hipStream_t st);
 int staged_d2h(void *host, const void *dev, size_t bytes, hipStream_t st);
 
-// batch = true: a plan whose passes run fused with other transforms' (the
-// batch table's schedule)
-int create_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, bool batch = false);
+int create_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use = ALONE);
 void clear_schedules();
 void clear_plan_cache();
-int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, bool batch = false);
+int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use = ALONE);
 
 }  // namespace gsn
 

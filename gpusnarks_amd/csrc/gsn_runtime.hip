@@ -129,20 +129,22 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
 // 136 / 249, 2^20 285 / 515, 2^22 1210 / 2280: a transform of 2^16 or 2^17
 // leaves most of the chip without a tile of 2^11.  Batches fill it, so there
 // everything from 2^15 goes this way (64 ragged transforms: 986 us; 998 with
-// 2^14 too, 1031 from 2^16, 1248 with none below 2^18).
-static std::vector<PassCfg> matrix_passes(int field, unsigned L, bool batch)
+// 2^14 too, 1031 from 2^16, 1248 with none below 2^18), except the few that
+// do not (FUSED_FEW, batch_uses).
+static std::vector<PassCfg> matrix_passes(int field, unsigned L, PlanUse use)
 {
     static const int R[][4] = {{5, 5, 5},    {5, 6, 5},    {6, 5, 6},    {6, 6, 6},    {5, 5, 4, 5},
                                {5, 5, 5, 5}, {6, 5, 5, 5}, {6, 5, 5, 6}, {6, 6, 5, 6}, {6, 6, 6, 6}};
     static const int DENSE[][3] = {{5, 5}, {6, 5}, {6, 6}, {4, 4, 5}, {4, 5, 5}, {5, 5, 5}};
     std::vector<PassCfg> v;
-    if (field != GSN_FIELD_FP32 && !batch && L >= 10 && L <= 15) {
+    if (field != GSN_FIELD_FP32 && use == ALONE && L >= 10 && L <= 15) {
         for (int r : DENSE[L - 10])
             if (r)
                 v.push_back({r, L == 15 ? 6 : 5, 1, MAT_DENSE});
         return v;
     }
-    if (field == GSN_FIELD_FP32 || L < 15 || L > 24 || (!batch && (L == 16 || L == 17)))
+    if (field == GSN_FIELD_FP32 || L < 15 || L > 24 || (use == ALONE && (L == 16 || L == 17)) ||
+        (use == FUSED_FEW && L < 18))
         return v;
     const int *r = R[L - 15], P = r[3] ? 4 : 3;
     for (int i = 0; i < P; ++i)
@@ -188,14 +190,14 @@ static void load_default_schedules()
 // Elsewhere the matrix passes go first where there are any (matrix_passes),
 // then the shipped table, then the defaults.  matrix = false: the schedule
 // of the vector kernels, which the tuning calls speak of.
-std::vector<PassCfg> choose_passes(int field, unsigned log_n, bool batch, bool matrix)
+std::vector<PassCfg> choose_passes(int field, unsigned log_n, PlanUse use, bool matrix)
 {
     static std::once_flag once;
     std::call_once(once, load_default_schedules);
     std::lock_guard<std::mutex> lk(g_tune_mutex);
     const std::pair<int, unsigned> key{field, log_n};
-    const std::vector<PassCfg> mat = matrix ? matrix_passes(field, log_n, batch) : std::vector<PassCfg>();
-    if (batch) {
+    const std::vector<PassCfg> mat = matrix ? matrix_passes(field, log_n, use) : std::vector<PassCfg>();
+    if (use != ALONE) {
         auto ib = g_tuned_batch.find(key);
         if (ib != g_tuned_batch.end())
             return ib->second;
@@ -537,7 +539,7 @@ int PlanImpl<GSN_FIELD_MNT6753_FR>::build_tables(const fields::ScalarMNT6 &w, si
 }
 
 template <int FID>
-static int create_plan_t(PlanBase **out, unsigned log_n, const void *omega, int inverse, bool batch)
+static int create_plan_t(PlanBase **out, unsigned log_n, const void *omega, int inverse, PlanUse use)
 {
     using Info = FieldInfo<FID>;
     using H = typename Info::Host;
@@ -558,20 +560,20 @@ static int create_plan_t(PlanBase **out, unsigned log_n, const void *omega, int 
     p->field = FID;
     p->log_n = log_n;
     p->inverse = inverse ? 1 : 0;
-    p->batch_mode = batch;
+    p->use = use;
     GSN_TRY(p->build(w));
     *out = p.release();
     return GSN_OK;
 }
 
-int create_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, bool batch)
+int create_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use)
 {
     if (!out)
         return set_error(GSN_ERR_INVALID_ARGUMENT, "plan pointer is NULL");
     switch (field) {
-    case GSN_FIELD_FP32: return create_plan_t<GSN_FIELD_FP32>(out, log_n, omega, inverse, batch);
-    case GSN_FIELD_MNT4753_FR: return create_plan_t<GSN_FIELD_MNT4753_FR>(out, log_n, omega, inverse, batch);
-    case GSN_FIELD_MNT6753_FR: return create_plan_t<GSN_FIELD_MNT6753_FR>(out, log_n, omega, inverse, batch);
+    case GSN_FIELD_FP32: return create_plan_t<GSN_FIELD_FP32>(out, log_n, omega, inverse, use);
+    case GSN_FIELD_MNT4753_FR: return create_plan_t<GSN_FIELD_MNT4753_FR>(out, log_n, omega, inverse, use);
+    case GSN_FIELD_MNT6753_FR: return create_plan_t<GSN_FIELD_MNT6753_FR>(out, log_n, omega, inverse, use);
     default: return set_error(GSN_ERR_INVALID_ARGUMENT, "unknown field id " + std::to_string(field));
     }
 }
@@ -623,13 +625,13 @@ void clear_plan_cache()
     g_plan_cache.clear();
 }
 
-int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, bool batch)
+int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use)
 {
     std::string key(16, '\0');
     std::memcpy(&key[0], &field, 4);
     std::memcpy(&key[4], &log_n, 4);
     std::memcpy(&key[8], &inverse, 4);
-    key[12] = batch ? 1 : 0;
+    key[12] = (char)use;
     if (omega)
         key.append((const char *)omega, element_bytes(field));
     std::lock_guard<std::mutex> lk(g_cache_mutex);
@@ -639,7 +641,7 @@ int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, in
         return GSN_OK;
     }
     PlanBase *p = nullptr;
-    GSN_TRY(create_plan(&p, field, log_n, omega, inverse, batch));
+    GSN_TRY(create_plan(&p, field, log_n, omega, inverse, use));
     g_plan_cache[key].reset(p);
     *out = p;
     return GSN_OK;
@@ -870,7 +872,7 @@ int gsn_tuning_get(int field, unsigned log_n, int *shapes, int max_passes, int *
 {
     if (!num_passes)
         return set_error(GSN_ERR_INVALID_ARGUMENT, "num_passes is NULL");
-    const std::vector<PassCfg> v = choose_passes(field, log_n, false, false);
+    const std::vector<PassCfg> v = choose_passes(field, log_n, ALONE, false);
     *num_passes = (int)v.size();
     if ((int)v.size() > max_passes || (!shapes && !v.empty()))
         return set_error(GSN_ERR_INVALID_ARGUMENT, "shapes buffer too small");

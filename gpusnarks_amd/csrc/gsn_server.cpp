@@ -154,7 +154,7 @@ int enqueue_single_t(PlanBase *base, const gsn_batch_item &it, Wave *w, hipStrea
 int enqueue_single(const gsn_batch_item &it, Wave *w, hipStream_t s)
 {
     PlanBase *p = nullptr;
-    GSN_TRY(cached_plan(&p, it.field, it.log_n, it.omega, it.inverse, true));
+    GSN_TRY(cached_plan(&p, it.field, it.log_n, it.omega, it.inverse, FUSED));
     switch (it.field) {
     case GSN_FIELD_FP32: return enqueue_single_t<GSN_FIELD_FP32>(p, it, w, s);
     case GSN_FIELD_MNT4753_FR: return enqueue_single_t<GSN_FIELD_MNT4753_FR>(p, it, w, s);
@@ -163,20 +163,23 @@ int enqueue_single(const gsn_batch_item &it, Wave *w, hipStream_t s)
 }
 
 // Device bytes a request needs in a wave: operand (host requests) +
-// workspace + job tables, each rounded to the allocator alignment.
+// workspace + job tables, each rounded to the allocator alignment; for the
+// larger of the schedules it may take there.
 size_t request_bytes(int field, unsigned log_n, bool device)
 {
     const size_t n = (size_t)1 << log_n, eb = element_bytes(field);
-    const std::vector<PassCfg> v = choose_passes(field, log_n, true);
-    const int nbuf = schedule_buffers(v);
-    size_t bytes = device ? 0 : align_up(n * eb);
-    bytes += align_up((size_t)nbuf * n * eb);
-    for (const PassCfg &c : v) {
-        const size_t tiles = (n >> c.log_r) >> c.log_w;
-        // a job table and a tile map per pass (worst case: a group of its own)
-        bytes += align_up(sizeof(PassJob<FMnt6>)) + align_up(tiles * sizeof(uint32_t));
+    size_t most = 0;
+    for (const PlanUse use : {FUSED, FUSED_FEW}) {
+        const std::vector<PassCfg> v = choose_passes(field, log_n, use);
+        size_t bytes = align_up((size_t)schedule_buffers(v) * n * eb);
+        for (const PassCfg &c : v) {
+            const size_t tiles = (n >> c.log_r) >> c.log_w;
+            // a job table and a tile map per pass (worst case: a group of its own)
+            bytes += align_up(sizeof(PassJob<FMnt6>)) + align_up(tiles * sizeof(uint32_t));
+        }
+        most = std::max(most, bytes);
     }
-    return bytes + ALIGN;
+    return (device ? 0 : align_up(n * eb)) + most + ALIGN;
 }
 
 }  // namespace

@@ -122,7 +122,7 @@ struct PlanImpl final : PlanBase {
     {
         const H w = inverse ? omega_fwd.mul_inv() : omega_fwd;
         const size_t n = (size_t)1 << log_n;
-        cfg = choose_passes(FID, log_n, batch_mode);
+        cfg = choose_passes(FID, log_n, use);
         num_passes = (int)cfg.size();
         workspace_buffers = schedule_buffers(cfg);
         for (const PassCfg &c : cfg)

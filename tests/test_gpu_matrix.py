@@ -87,3 +87,29 @@ def test_dense_passes_match_vector_kernels(field, log_n):
             g.tuning_clear()
             g.tuning_load(shipped)  # the default routes again
         assert np.array_equal(got, want) and np.array_equal(again, want_again), (field, log_n, inverse)
+
+
+# launches of a batch: two passes on the vector kernels; on the matrix cores
+# three passes, each with a launch per radix
+@pytest.mark.parametrize("sizes,launches", [((16,), 2), ((17,), 2), ((16, 16), 2), ((15, 16), 2), ((15, 15, 16), 2),
+                                            ((16, 17), 2), ((15, 16, 17), 2), ((16, 16, 17), 2),
+                                            ((15, 15, 16, 16, 16, 17), 2), ((15,), 3), ((15, 15, 15, 15), 3),
+                                            ((16, 16, 16), 3), ((17, 17), 3), ((18,), 3), ((15, 16, 16), 4),
+                                            ((15, 15, 16, 16, 17, 17), 6), ((16, 17, 18), 6)])
+def test_small_batches_take_the_faster_kernels(sizes, launches):
+    """Batches on both sides of the line between vector kernels and matrix
+    passes, every transform bit-identical to its plan alone."""
+    field = g.FIELD_MNT6753_FR
+    print("small batch", sizes, flush=True)
+    xs = [operands(field, l, 0xBA7 + 31 * i + l) for i, l in enumerate(sizes)]
+    d_in = [g.DeviceArray.from_numpy(x) for x in xs]
+    d_out = [g.DeviceArray(x.nbytes) for x in xs]
+    batch = g.Batch([(field, l, i % 2 == 1, a.ptr, b.ptr) for i, (l, a, b) in enumerate(zip(sizes, d_in, d_out))])
+    assert batch.num_launches == launches
+    batch.launch()
+    g.synchronize()
+    for i, (l, x, d) in enumerate(zip(sizes, xs, d_out)):
+        plan = g.Plan(field, l, inverse=i % 2 == 1)
+        assert np.array_equal(d.download(x.shape), run(plan, x, in_place=False)), (sizes, i)
+        plan.close()
+    batch.close()
