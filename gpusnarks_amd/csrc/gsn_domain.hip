@@ -410,14 +410,19 @@ int build_matrices(DeviceBuffer &mat, const std::vector<TW753> &records)
 
 struct CosetTables {
     DeviceBuffer lo, hi;
-    DeviceBuffer mat;  // hi as byte matrices (coset_matrix)
+    DeviceBuffer mat;  // hi as byte matrices (coset_matrix), or empty
     uint32_t h = 0;
+    bool matrix() const { return mat.ptr != nullptr; }
     CosetArgs args() const { return CosetArgs{(const TW753 *)lo.ptr, mat.ptr, h}; }
 };
 // Whether hi's products go to the matrix cores: 64 consecutive i share one
 // from 2^11 points (7.0 against 8.9 us there, 95 against 117 at 2^20).  These
 // tables outlive the calls, and at 9216 B a power (224 as a record) they would
-// pass 10 MB each beyond 2^20.
+// pass 10 MB each beyond 2^20.  All of them together stay below
+// COSET_MATRIX_BYTES, 13 generators' and directions' worth at 2^20; those that
+// come after it, or find no memory, keep to the records.  (What is built is
+// kept: a captured graph may hold its address.)
+constexpr size_t COSET_MATRIX_BYTES = (size_t)128 << 20;
 template <int FID>
 constexpr bool coset_matrix(unsigned log_n)
 {
@@ -426,6 +431,7 @@ constexpr bool coset_matrix(unsigned log_n)
 
 std::mutex g_coset_mutex;
 std::map<std::tuple<int, unsigned, int, std::vector<uint32_t>>, std::unique_ptr<CosetTables>> g_coset;
+size_t g_coset_matrix_bytes = 0;
 
 // g^(+-i) = lo[i & (2^h - 1)] * hi[i >> h] for i < 2^log_n
 template <int FID>
@@ -457,9 +463,19 @@ int coset_tables(CosetTables **out, const typename FieldInfo<FID>::Host &g, unsi
         GSN_TRY(t->hi.alloc(nhi * sizeof(tw)));
         GSN_TRY(hip_status(hipMemcpy(t->lo.ptr, lo.data(), nlo * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
         GSN_TRY(hip_status(hipMemcpy(t->hi.ptr, hi.data(), nhi * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
-        if constexpr (FID != GSN_FIELD_FP32)
-            if (coset_matrix<FID>(log_n))
-                GSN_TRY(build_matrices<FID>(t->mat, hi));
+        if constexpr (FID != GSN_FIELD_FP32) {
+            const size_t bytes = nhi * MAT_BYTES;
+            if (coset_matrix<FID>(log_n) && g_coset_matrix_bytes + bytes <= COSET_MATRIX_BYTES) {
+                const int st = build_matrices<FID>(t->mat, hi);
+                if (st == GSN_ERR_OUT_OF_MEMORY) {
+                    t->mat = DeviceBuffer();
+                    (void)hipGetLastError();
+                } else {
+                    GSN_TRY(st);
+                    g_coset_matrix_bytes += bytes;
+                }
+            }
+        }
         slot = std::move(t);
     }
     *out = slot.get();
@@ -488,7 +504,7 @@ int coset_t(void *out, const void *in, size_t n, const void *g_limbs, int invers
     CosetTables *t = nullptr;
     GSN_TRY(coset_tables<FID>(&t, g, log_n, inverse));
     if constexpr (FID != GSN_FIELD_FP32) {
-        if (coset_matrix<FID>(log_n)) {
+        if (t->matrix()) {
             launch_coset753<F>((E753 *)out, (const E753 *)in, t->args(), n, st);
             return hip_status(hipGetLastError(), "coset launch");
         }
@@ -563,7 +579,7 @@ struct ExtPlan : PlanBase {
     PlanBase *half = nullptr;
     CosetTables *tab = nullptr;  // g^i (forward) or g^-i (inverse), i < m
     typename F::tw_t c;          // G (forward) or 1 / (1 - G) (inverse)
-    DeviceBuffer cmat;           // its matrix (coset_matrix)
+    DeviceBuffer cmat;           // its matrix, where tab has them
     std::unique_ptr<BatchImpl> halves;  // both half transforms, fused
     const void *halves_in = nullptr;
     void *halves_out = nullptr;
@@ -596,7 +612,7 @@ struct ExtPlan : PlanBase {
     bool matrix_step(const void *in, void *out, size_t m, hipStream_t st)
     {
         if constexpr (FID != GSN_FIELD_FP32) {
-            if (coset_matrix<FID>(log_n - 1)) {
+            if (tab->matrix()) {
                 launch_ext753<F>((E753 *)out, (const E753 *)in, tab->args(), cmat.ptr, m, inverse, st);
                 return true;
             }
@@ -617,7 +633,7 @@ struct ExtPlan : PlanBase {
         GSN_TRY(coset_tables<FID>(&tab, g, lm, inv));
         c = inv ? record<FID>((H::one() - G).mul_inv()) : record<FID>(G);
         if constexpr (FID != GSN_FIELD_FP32)
-            if (coset_matrix<FID>(lm))
+            if (tab->matrix())
                 GSN_TRY(build_matrices<FID>(cmat, {c}));
         num_passes = half->num_passes + 1;  // the halves' passes are fused
         device_bytes = half->device_bytes;

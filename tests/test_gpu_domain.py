@@ -421,3 +421,28 @@ def test_mixed_radix_errors():
         g.Plan.mixed(g.FIELD_MNT4753_FR, 1575 * 2)  # 3^2 does not divide p - 1 of MNT4-753 Fr
     with pytest.raises(g.GsnError):
         g.Plan.mixed(g.FIELD_MNT4753_FR, 3 << 16)  # 2^16 exceeds the 2-adicity
+
+
+def test_coset_tables_of_many_generators_stay_bounded():
+    """24 generators at 2^20, whose matrices would take 237 MB: device memory
+    grows by at most the matrices' bound (128 MiB) and the records, and the
+    shifts past it stay right."""
+    field, log_n = g.FIELD_MNT6753_FR, 20
+    n, p = 1 << log_n, g.MODULI[field]
+    x = np.concatenate([residues(field, 1 << 10, 0xC05E7)] * (n >> 10))
+    d_in, d_out = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+    at = [0, 1, 63, 64, 1023, 1024, 65537, n - 64, n - 1]
+    g.synchronize()
+    free = g.device_memory()[0]
+    for i in range(24):
+        say("coset generator", i)
+        shift = 1000003 + 2 * i
+        rep = shift * (1 << 768) % p
+        g.coset_shift(field, d_out.ptr, d_in.ptr, n, np.array([(rep >> (32 * k)) & 0xFFFFFFFF for k in range(24)],
+                                                             dtype=np.uint32))
+        got = d_out.download(x.shape)
+        for k in at:
+            want = sum(int(v) << (32 * j) for j, v in enumerate(x[k])) * pow(shift, k, p) % p
+            assert sum(int(v) << (32 * j) for j, v in enumerate(got[k])) == want, (i, k)
+    used = free - g.device_memory()[0]
+    assert used <= (128 << 20) + 24 * (1 << 20), used
