@@ -4,9 +4,11 @@ For each (field, log2 n) it enumerates pass schedules -- how log2 n splits
 into passes (the radix of each pass), how many columns a tile holds (tile
 depth; for the 753-bit field also the workgroup size: 64, 128 or 256
 threads) and the register radix -- times every candidate on the GPU with
-HIP events, checks that its output is bit-identical to the default
-schedule's, and writes the fastest per size to tuning.txt beside the
-library, which the library reads at start-up.
+HIP events, checks that its output is bit-identical to the library's own
+choice, and writes the fastest per size to tuning.txt beside the library,
+which the library reads at start-up.  Schedules are those of the vector
+kernels: a size whose own choice (the matrix cores, for most 753-bit sizes)
+is faster than all of them gets no line.
 
     python3 -m gpusnarks_amd.autotune [--fields mnt6,fp32] [--out PATH]
 """
@@ -75,8 +77,10 @@ SETTLE_MS = 50.0
 def time_schedule(field, log_n, sched, x_dev, y_dev, stream, reps, settle_ms=SETTLE_MS):
     """Mean time of one transform under `sched`: untimed transforms until
     `settle_ms` of GPU time has passed, then at least `reps` timed back to
-    back (more for short transforms, so the timed region lasts ~10 ms)."""
-    g.tuning_set(field, log_n, sched)
+    back (more for short transforms, so the timed region lasts ~10 ms).
+    None: the library's own choice."""
+    if sched is not None:
+        g.tuning_set(field, log_n, sched)
     plan = g.Plan(field, log_n)
     e0, e1 = g.Event(), g.Event()
 
@@ -112,6 +116,7 @@ def tune(fields, sizes=None, budget_s=60.0, log=print):
             g.tuning_clear()
             ref = g.best_fft(x, None, field)
             default = g.tuning_get(field, log_n)
+            g.tuning_clear()  # a schedule that was reported can be set like any other
             cands = candidates(field, log_n)
             if default not in cands:
                 cands.insert(0, default)
@@ -131,11 +136,15 @@ def tune(fields, sizes=None, budget_s=60.0, log=print):
                 if best is None or ms < best[0]:
                     best = (ms, sched)
             g.tuning_clear()
-            ms_default = time_schedule(field, log_n, default, x_dev, y_dev, stream, reps)
+            ms_default = time_schedule(field, log_n, None, x_dev, y_dev, stream, reps)
             g.tuning_clear()
-            results[(field, log_n)] = (best[1], best[0], ms_default)
-            log("%s 2^%d: best %s %.4f ms (default %s %.4f ms, %d candidates)"
-                % (name, log_n, best[1], best[0], default, ms_default, len(cands)))
+            if best is not None and best[0] < ms_default:
+                results[(field, log_n)] = (best[1], best[0], ms_default)
+            else:
+                results[(field, log_n)] = (None, ms_default, ms_default)
+            log("%s 2^%d: %s %.4f ms (default %.4f ms, %d candidates)"
+                % (name, log_n, results[(field, log_n)][0] or "the library's choice", results[(field, log_n)][1],
+                   ms_default, len(cands)))
     return results
 
 
@@ -163,12 +172,15 @@ def kept_lines(path, results):
 
 
 def write_table(results, path, keep_from=None):
-    """Tuned sizes from `results`, the other sizes and the batch lines as
-    the existing table (`keep_from`, else `path`) has them."""
+    """Tuned sizes from `results` (none for the library's choice), the other
+    sizes and the batch lines as the existing table (`keep_from`, else `path`)
+    has them."""
     lines = ["# field log_n  log_r,log_w,log_e per pass  (written by gpusnarks_amd.autotune)",
              "# 'batch field log_n ...': the schedule of transforms fused into batches, where it differs"]
     rows = kept_lines(keep_from or path, results)
     for (field, log_n), (sched, ms, ms_default) in results.items():
+        if sched is None:
+            continue
         rows[(field, log_n)] = ("%d %d %s  # %.4f ms (default %.4f ms)"
                                 % (field, log_n, " ".join("%d,%d,%d" % s for s in sched), ms, ms_default))
     lines += [rows[k] for k in sorted(rows)]

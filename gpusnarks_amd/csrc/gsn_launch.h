@@ -61,6 +61,10 @@ enum : int { MAT_FIRST = 1, MAT_MID = 2, MAT_LAST = 3, MAT_MID2 = 4, MAT_DENSE =
 struct PassCfg {
     int log_r, log_w, log_e;
     int kind = 0;
+    bool operator==(const PassCfg &o) const
+    {
+        return log_r == o.log_r && log_w == o.log_w && log_e == o.log_e && kind == o.kind;
+    }
 };
 
 // Workspace buffers of n elements a schedule needs: Stockham passes write

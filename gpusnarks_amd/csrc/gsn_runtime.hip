@@ -21,6 +21,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <set>
 #include <string>
 #include <vector>
 
@@ -158,9 +159,17 @@ using Schedules = std::map<std::pair<int, unsigned>, std::vector<PassCfg>>;
 // schedules set by the program or its own tuning file, and those of the
 // table beside the library; batch: overrides for fused launches
 Schedules g_tuned, g_tuned_batch, g_shipped, g_shipped_batch;
+// what that table says, whether it is in use or not
+Schedules g_table, g_table_batch;
+// sizes whose schedule gsn_tuning_get reported while no program had set one
+std::set<std::pair<int, unsigned>> g_reported;
+
+// Where a schedule comes from: gsn_tuning_set, a table of the program's, the
+// table beside the library, or that table while another one is in use.
+enum class Origin { PROGRAM, TABLE, SHIPPED, UNUSED };
 }  // namespace
 
-int load_schedules(const char *path, bool shipped);
+static int load_schedules(const char *path, Origin from);
 
 // tuning.txt beside the library
 static std::string shipped_table()
@@ -177,16 +186,23 @@ static std::string shipped_table()
 static void load_default_schedules()
 {
     const char *env = std::getenv("GSN_TUNING_FILE");
-    if (env && *env) {
-        load_schedules(env, false);
-        return;
-    }
+    const bool other = env && *env;
     const std::string p = shipped_table();
     if (!p.empty() && std::ifstream(p).good())
-        load_schedules(p.c_str(), true);
+        load_schedules(p.c_str(), other ? Origin::UNUSED : Origin::SHIPPED);
+    if (other)
+        load_schedules(env, Origin::TABLE);
 }
 
-// A schedule that the program set, or read from a table of its own, stands.
+// the vector kernels' schedule of a transform alone that nobody has set one for
+static std::vector<PassCfg> vector_schedule(const std::pair<int, unsigned> &key)
+{
+    const auto it = g_shipped.find(key);
+    return it != g_shipped.end() ? it->second : default_passes(key.first, key.second);
+}
+
+// A schedule that the program set, or read from a table of its own, stands; a
+// transform in a batch takes the batch lines' first, of either table.
 // Elsewhere the matrix passes go first where there are any (matrix_passes),
 // then the shipped table, then the defaults.  matrix = false: the schedule
 // of the vector kernels, which the tuning calls speak of.
@@ -208,12 +224,7 @@ std::vector<PassCfg> choose_passes(int field, unsigned log_n, PlanUse use, bool 
     auto it = g_tuned.find(key);
     if (it != g_tuned.end())
         return it->second;
-    if (!mat.empty())
-        return mat;
-    it = g_shipped.find(key);
-    if (it != g_shipped.end())
-        return it->second;
-    return default_passes(field, log_n);
+    return mat.empty() ? vector_schedule(key) : mat;
 }
 
 static int validate_schedule(int field, unsigned log_n, const std::vector<PassCfg> &v)
@@ -240,17 +251,36 @@ static int validate_schedule(int field, unsigned log_n, const std::vector<PassCf
     return GSN_OK;
 }
 
-int set_schedule(int field, unsigned log_n, const std::vector<PassCfg> &v, bool batch = false, bool shipped = false)
+// The shipped table's line, also as another table repeats it, and the schedule
+// that gsn_tuning_get reported as the library's own leave the choice to the
+// library, whose matrix passes have no schedule to report.
+static int set_schedule(int field, unsigned log_n, const std::vector<PassCfg> &v, bool batch, Origin from)
 {
     GSN_TRY(validate_schedule(field, log_n, v));
     std::lock_guard<std::mutex> lk(g_tune_mutex);
-    if (shipped) {  // loading it again restores what it says
-        (batch ? g_tuned_batch : g_tuned).erase({field, log_n});
-        (batch ? g_shipped_batch : g_shipped)[{field, log_n}] = v;
+    const std::pair<int, unsigned> key{field, log_n};
+    Schedules &tuned = batch ? g_tuned_batch : g_tuned, &table = batch ? g_table_batch : g_table;
+    if (from == Origin::SHIPPED || from == Origin::UNUSED)
+        table[key] = v;
+    if (from == Origin::UNUSED)
+        return GSN_OK;
+    const auto line = table.find(key);
+    if (from == Origin::SHIPPED || (from == Origin::TABLE && line != table.end() && line->second == v)) {
+        tuned.erase(key);
+        (batch ? g_shipped_batch : g_shipped)[key] = v;
+    } else if (from == Origin::PROGRAM && g_reported.count(key) && v == vector_schedule(key)) {
+        tuned.erase(key);
     } else {
-        (batch ? g_tuned_batch : g_tuned)[{field, log_n}] = v;
+        tuned[key] = v;
     }
     return GSN_OK;
+}
+
+static void report_schedule(int field, unsigned log_n)
+{
+    std::lock_guard<std::mutex> lk(g_tune_mutex);
+    if (!g_tuned.count({field, log_n}))
+        g_reported.insert({field, log_n});
 }
 
 void clear_schedules()
@@ -260,11 +290,12 @@ void clear_schedules()
     g_tuned_batch.clear();
     g_shipped.clear();
     g_shipped_batch.clear();
+    g_reported.clear();
 }
 
 // "field log_n r,w,e r,w,e ..." per line, "batch field log_n ..." for the
 // schedule of transforms fused into batches; '#' starts a comment
-int load_schedules(const char *path, bool shipped)
+static int load_schedules(const char *path, Origin from)
 {
     std::ifstream f(path);
     if (!f.good())
@@ -298,7 +329,7 @@ int load_schedules(const char *path, bool shipped)
                                                                ": bad pass shape '" + tok + "'");
             v.push_back(c);
         }
-        GSN_TRY(set_schedule(field, log_n, v, batch, shipped));
+        GSN_TRY(set_schedule(field, log_n, v, batch, from));
     }
     return GSN_OK;
 }
@@ -863,7 +894,7 @@ int gsn_tuning_set(int field, unsigned log_n, const int *shapes, int num_passes)
     for (int i = 0; i < num_passes; ++i)
         v.push_back({shapes[3 * i], shapes[3 * i + 1], shapes[3 * i + 2]});
     (void)choose_passes(field, log_n);  // load the default file first, so it cannot override this
-    GSN_TRY(set_schedule(field, log_n, v));
+    GSN_TRY(set_schedule(field, log_n, v, false, Origin::PROGRAM));
     clear_plan_cache();
     return GSN_OK;
 }
@@ -881,6 +912,7 @@ int gsn_tuning_get(int field, unsigned log_n, int *shapes, int max_passes, int *
         shapes[3 * i + 1] = v[i].log_w;
         shapes[3 * i + 2] = v[i].log_e;
     }
+    report_schedule(field, log_n);
     return GSN_OK;
 }
 
@@ -900,7 +932,7 @@ int gsn_tuning_load(const char *path)
     // the shipped table by name restores the defaults
     char a[PATH_MAX], b[PATH_MAX];
     const bool shipped = realpath(path, a) && realpath(shipped_table().c_str(), b) && std::strcmp(a, b) == 0;
-    GSN_TRY(load_schedules(path, shipped));
+    GSN_TRY(load_schedules(path, shipped ? Origin::SHIPPED : Origin::TABLE));
     clear_plan_cache();
     return GSN_OK;
 }

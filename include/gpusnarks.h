@@ -267,11 +267,15 @@ int gsn_msm(gsn_msm_bases *bases, void *d_out, const void *d_scalars, void *stre
  * use, by batches or by calls running on other threads, stay valid).  At
  * start-up the library reads tuning.txt beside itself (or $GSN_TUNING_FILE):
  * lines "field log_n r,w,e r,w,e ...", and "batch field log_n ..." for the
- * schedule of transforms fused into batches.  Schedules are those of the
- * vector kernels.  The larger 753-bit sizes run on the matrix cores instead,
- * with passes of their own, unless gsn_tuning_set or a table other than the
- * one beside the library names a schedule for them; gsn_tuning_get reports
- * the vector kernels' schedule either way. */
+ * schedule of transforms fused into batches, which goes before the other one
+ * there.  Schedules are those of the vector kernels.  The larger 753-bit sizes
+ * run on the matrix cores instead, with passes of their own, unless
+ * gsn_tuning_set or a table other than the one beside the library names a
+ * schedule for them (in batches: where the table beside the library has no
+ * batch line for the size); gsn_tuning_get reports the vector kernels' schedule
+ * either way.  Setting what gsn_tuning_get reported while the library chose
+ * gives the choice back to it, and so does a table's line that repeats the one
+ * beside the library; gsn_tuning_clear forgets what was reported. */
 int gsn_tuning_set(int field, unsigned log_n, const int *shapes, int num_passes);
 int gsn_tuning_get(int field, unsigned log_n, int *shapes, int max_passes, int *num_passes);
 int gsn_tuning_clear(void);

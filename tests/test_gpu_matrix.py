@@ -113,3 +113,99 @@ def test_small_batches_take_the_faster_kernels(sizes, launches):
         assert np.array_equal(d.download(x.shape), run(plan, x, in_place=False)), (sizes, i)
         plan.close()
     batch.close()
+
+
+def test_schedules_go_back_to_the_library():
+    """A schedule that is read, replaced and put back leaves the size on the
+    library's own choice, and so does a table that repeats the shipped lines
+    beside others; a schedule of the program's own stands."""
+    field = g.FIELD_MNT6753_FR
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+
+    def passes(f, log_n):
+        plan = g.Plan(f, log_n)
+        try:
+            return plan.num_passes
+        finally:
+            plan.close()
+
+    try:
+        g.tuning_clear()
+        g.tuning_load(shipped)
+        vector = [(9, 1, 1), (9, 1, 1)]
+        own = {(field, 18): 3, (field, 20): 4, (g.FIELD_MNT4753_FR, 13): 3}
+        for (f, l), p in own.items():
+            assert passes(f, l) == p
+        # the program's own schedule, even the vector kernels' shipped one
+        g.tuning_set(field, 18, vector)
+        assert passes(field, 18) == 2
+        g.tuning_clear()
+        g.tuning_load(shipped)
+        for (f, l), p in own.items():
+            before = g.tuning_get(f, l)
+            g.tuning_set(f, l, before)
+            assert passes(f, l) == p and g.tuning_get(f, l) == before
+            g.tuning_set(f, l, [(7, 0, 1)] * (l // 7) + [(l % 7, 2, 1)])
+            assert passes(f, l) == l // 7 + 1
+            g.tuning_set(f, l, before)
+            assert passes(f, l) == p and g.tuning_get(f, l) == before
+    finally:
+        g.tuning_clear()
+        g.tuning_load(shipped)
+
+
+def test_tables_that_repeat_shipped_lines(tmp_path):
+    field = g.FIELD_MNT6753_FR
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+    lines = open(shipped).read().splitlines()
+    copy, mine = tmp_path / "copy.txt", tmp_path / "mine.txt"
+    copy.write_text("\n".join("0 20 10,4,4 10,4,4" if l.startswith("0 20 ") else l for l in lines) + "\n")
+    mine.write_text("2 18 9,0,1 9,0,1\nbatch 2 15 8,0,1 7,0,1\n")
+    x = g.DeviceArray(96 << 18)
+
+    def passes():
+        plan, batch = g.Plan(field, 18), g.Batch([(field, 15, False, x.ptr, x.ptr)])
+        out = plan.num_passes, batch.num_launches
+        plan.close()
+        batch.close()
+        return out
+
+    try:
+        g.tuning_clear()
+        g.tuning_load(shipped)
+        assert passes() == (3, 3)
+        g.tuning_load(str(copy))
+        assert g.tuning_get(g.FIELD_FP32, 20) == [(10, 4, 4), (10, 4, 4)]
+        assert passes() == (3, 3) and g.tuning_get(field, 18) == [(9, 1, 1), (9, 1, 1)]
+        g.tuning_load(str(mine))
+        assert passes() == (2, 2)
+        g.tuning_load(str(copy))  # the shipped lines again
+        assert passes() == (3, 3)
+    finally:
+        g.tuning_clear()
+        g.tuning_load(shipped)
+
+
+def test_autotuner_leaves_faster_choices_to_the_library(tmp_path):
+    """At MNT6 2^10 no schedule of the vector kernels is near the matrix cores:
+    the tuner writes no line, and its table keeps the library's choice."""
+    from gpusnarks_amd import autotune as at
+    field = g.FIELD_MNT6753_FR
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+    table = tmp_path / "t.txt"
+    try:
+        results = at.tune(["mnt6"], [10], budget_s=2.0, log=lambda *a: print(*a, flush=True))
+        sched, ms, ms_default = results[(field, 10)]
+        assert sched is None and ms == ms_default
+        at.write_table(results, str(table), keep_from=shipped)
+        assert not any(l.startswith("2 10 ") for l in table.read_text().splitlines())
+        g.tuning_clear()
+        g.tuning_load(shipped)
+        g.tuning_load(str(table))
+        for l, p in ((10, 2), (15, 3), (18, 3), (20, 4)):
+            plan = g.Plan(field, l)
+            assert plan.num_passes == p
+            plan.close()
+    finally:
+        g.tuning_clear()
+        g.tuning_load(shipped)

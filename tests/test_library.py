@@ -196,3 +196,12 @@ def test_autotuner_candidates_and_table_merge(tmp_path):
     finally:
         g.tuning_clear()
         g.tuning_load(os.path.join(os.path.dirname(g.library_path), "tuning.txt"))
+
+
+def test_table_has_no_line_for_the_librarys_choice(tmp_path):
+    from gpusnarks_amd import autotune as at
+    old, new = tmp_path / "old.txt", tmp_path / "new.txt"
+    old.write_text("0 20 6,4,4 6,4,4 8,4,4\n2 10 5,2,1 5,2,1\nbatch 2 10 5,2,1 5,2,1\n")
+    at.write_table({(g.FIELD_MNT6753_FR, 10): (None, 0.016, 0.016)}, str(new), keep_from=str(old))
+    rows = [l for l in new.read_text().splitlines() if not l.startswith("#")]
+    assert rows == ["0 20 6,4,4 6,4,4 8,4,4", "batch 2 10 5,2,1 5,2,1"]
