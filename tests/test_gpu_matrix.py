@@ -1,7 +1,7 @@
 """GPU: the 753-bit matrix passes against the vector kernels, bit for bit, at
-every schedule they have (three and four passes, 2^15 to 2^22), forward and
+every schedule they have (three and four passes, 2^15 to 2^24), forward and
 inverse, in place, with operands at the ends of the field, alone and (from
-2^15) in a batch."""
+2^15) in a batch; which calls take them."""
 import os
 import sys
 
@@ -209,3 +209,35 @@ def test_autotuner_leaves_faster_choices_to_the_library(tmp_path):
     finally:
         g.tuning_clear()
         g.tuning_load(shipped)
+
+
+@pytest.mark.parametrize("log_n", [23, 24])
+def test_largest_matrix_passes_match_vector_kernels(log_n):
+    """The two largest schedules, in place, and out of place in a batch."""
+    field = g.FIELD_MNT6753_FR
+    x = operands(field, log_n, 0x3A7 + log_n)
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+    for inverse in (False, True):
+        print("largest matrix passes", log_n, inverse, flush=True)
+        plan = g.Plan(field, log_n, inverse=inverse)
+        assert plan.num_passes == 4
+        got = run(plan, x, in_place=True)
+        plan.close()
+        d_in, d_out = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+        batch = g.Batch([(field, log_n, inverse, d_in.ptr, d_out.ptr)])
+        batch.launch()
+        g.synchronize()
+        assert np.array_equal(d_out.download(x.shape), got), (log_n, inverse)
+        batch.close()
+        print("vector kernels", log_n, inverse, flush=True)
+        try:
+            g.tuning_set(field, log_n, [(5, 2, 1)] * 4 + [(log_n - 20, 2, 1)])
+            plan = g.Plan(field, log_n, inverse=inverse)
+            assert plan.num_passes == 5
+            want = run(plan, x, in_place=False)
+            plan.close()
+        finally:
+            g.tuning_clear()
+            g.tuning_load(shipped)  # the default routes again
+        assert np.array_equal(got, want), (log_n, inverse)
+        del got, want

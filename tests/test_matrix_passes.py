@@ -1,7 +1,7 @@
 """The 753-bit matrix passes (gpusnarks_amd/csrc/matrix753_kernels.h) restated
 in Python, CPU only: their arithmetic with whole numbers at the ends of its
 ranges, and their digits, twiddle factors and addresses over a small prime
-field against the O(n^2) DFT."""
+field against the O(n^2) DFT, and the addresses of every schedule in use."""
 import random
 
 import numpy as np
@@ -187,3 +187,64 @@ def test_dense_sums_and_bounds(field):
             exact += want
         y = sum(parts) + 3 * p
         assert 0 < y < TOP and (y - exact) % p == 0
+
+
+SCHEDULES = {15: (5, 5, 5), 16: (5, 6, 5), 17: (6, 5, 6), 18: (6, 6, 6), 19: (5, 5, 4, 5), 20: (5, 5, 5, 5),
+             21: (6, 5, 5, 5), 22: (6, 5, 5, 6), 23: (6, 6, 5, 6), 24: (6, 6, 6, 6)}
+
+
+@pytest.mark.parametrize("log_n", sorted(SCHEDULES))
+def test_addresses_and_entries_of_every_schedule(log_n):
+    """MatTile's addresses of every tile, row and column: each pass reads and
+    writes every element once, the ones between the first and the last where
+    they read, with matrix entries inside the tables built for the pass and
+    32-bit arithmetic where the kernel has it."""
+    radices = SCHEDULES[log_n]
+    n, num, rp, n1 = 1 << log_n, len(radices), radices[-1], radices[0]
+    assert sum(radices) == log_n
+    W, u32 = 32, 1 << 32
+
+    def covers(at):
+        assert at.min() >= 0 and at.max() < n and at.size == n
+        seen = np.zeros(n, dtype=bool)
+        seen[at.reshape(-1)] = True
+        return seen.all()
+
+    log_ns = 0
+    for i, r in enumerate(radices):
+        R, log_g, log_s = 1 << r, radices[i - 1] if i else 0, log_n - log_ns - r
+        blk = np.arange(n >> (r + 5), dtype=np.int64)
+        row, col = np.arange(R)[None, :, None], np.arange(W)[None, None, :]
+        if i == 0:
+            kap = np.zeros_like(blk)
+            at = (blk * W)[:, None, None] + row * (n >> r) + col
+            assert covers(at)
+        elif i < num - 1:
+            log_hi = log_n - r - log_s - log_g
+            assert log_hi >= 0 and log_s >= rp >= 5
+            p, lo = blk >> (log_s - 5), (blk << 5) & ((1 << log_s) - 1)
+            assert (blk << 5).max() < u32
+            kap = p >> log_hi
+            pre = ((p & ((1 << log_hi) - 1)) << log_g) | kap
+            top, nxt = lo & ((1 << rp) - 1), lo >> rp
+            at = ((pre << (log_s + r)) + lo)[:, None, None] + (row << log_s) + col
+            assert covers(at)
+            # column factors: entry (kap << rp) + top + column of 2^(g + rp)
+            assert ((kap << rp) + top + W - 1).max() < 1 << (log_g + rp)
+            if i == num - 3:  # the pair (1, 3): 2 entries of 2^(g + r3)
+                assert log_s - rp == radices[2]
+                assert (2 * ((kap << (log_s - rp)) + nxt) + 1).max() < 2 << (log_g + radices[2])
+            else:
+                assert num == 3 or i == 2
+        else:
+            rev, k1 = blk >> (n1 - 5), (blk << 5) & ((1 << n1) - 1)
+            log_k = log_n - n1 - r - log_g
+            kap = rev >> log_k
+            mid = ((rev & ((1 << log_k) - 1)) << log_g) | kap if log_k else rev
+            assert covers((k1 * (n >> n1) + (mid << r))[:, None, None] + row + col * (n >> n1))
+            assert covers(((rev << n1) + k1)[:, None, None] + row * (n >> r) + col)
+        # step s takes entry ((2^s - 1) << g) + (kap << s) + kk, kk < 2^s
+        s = r - 1
+        assert kap.min() >= 0 and kap.max() < 1 << log_g
+        assert (((1 << s) - 1) << log_g) + (kap.max() << s) + (1 << s) - 1 < ((1 << r) - 1) << log_g
+        log_ns += r
