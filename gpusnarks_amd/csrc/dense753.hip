@@ -222,28 +222,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void d
     }
 }
 
-// matrices of w_n^(i mul), a block each
+// matrices of w_n^(i mul), i < entries
 template <class F>
-__global__ __launch_bounds__(128) void build_dense753_kernel(uint4 *out, const E753 *hi, const TW753 *lo, uint32_t h,
-                                                            uint64_t mul)
+__global__ __launch_bounds__(64) void build_dense753_kernel(uint4 *out, uint32_t entries, const E753 *hi,
+                                                           const TW753 *lo, uint32_t h, uint32_t log_n, uint64_t mul)
 {
-    __shared__ __align__(16) uint8_t img[MAT_BYTES];
-    matrix_image<F>(img, root_power<F>(hi, lo, h, (size_t)blockIdx.x * mul), threadIdx.x);
-    __syncthreads();
-    for (uint32_t q = threadIdx.x; q < MAT_BYTES / 16; q += 128)
-        out[(size_t)blockIdx.x * (MAT_BYTES / 16) + q] = reinterpret_cast<const uint4 *>(img)[q];
+    write_matrices<F>(out, entries, [&](uint32_t i) { return root_power<F>(hi, lo, h, log_n, i * mul); });
 }
 // records of w_n^(j c mul) at (j << log_c) + c, times scale if use_scale
 template <class F>
 __global__ __launch_bounds__(64) void build_dense753_records_kernel(TW753 *out, uint32_t count, const E753 *hi,
-                                                                    const TW753 *lo, uint32_t h, uint32_t log_c,
-                                                                    uint64_t mul, TW753 scale, int use_scale)
+                                                                    const TW753 *lo, uint32_t h, uint32_t log_n,
+                                                                    uint32_t log_c, uint64_t mul, TW753 scale, int use_scale)
 {
     const uint32_t i = blockIdx.x * 64 + threadIdx.x;
     if (i >= count)
         return;
     const size_t j = i >> log_c, c = i & ((1u << log_c) - 1u);
-    E753 v = root_power<F>(hi, lo, h, j * c * mul);
+    E753 v = root_power<F>(hi, lo, h, log_n, j * c * mul);
     if (use_scale)
         v = F::canon(F::mul(v, scale));
     out[i] = F::make_tw(v);
@@ -278,12 +274,12 @@ void launch_build_dense753(uint4 *mat, uint32_t log_r, TW753 *rec, uint32_t log_
 {
     const TW753 one{};
     if (mat)
-        hipLaunchKernelGGL(build_dense753_kernel<F>, dim3(1u << log_r), dim3(128), 0, st, mat, hi, lo, h,
-                           (uint64_t)1 << (log_n - log_r));
+        hipLaunchKernelGGL(build_dense753_kernel<F>, dim3(mat_blocks(1u << log_r)), dim3(64), 0, st, mat, 1u << log_r,
+                           hi, lo, h, log_n, (uint64_t)1 << (log_n - log_r));
     if (rec) {
         const uint32_t count = 1u << (log_s + log_next);
         hipLaunchKernelGGL(build_dense753_records_kernel<F>, dim3((count + 63) / 64), dim3(64), 0, st, rec, count, hi,
-                           lo, h, log_s, (uint64_t)1 << (log_n - log_s - log_next), scale ? *scale : one,
+                           lo, h, log_n, log_s, (uint64_t)1 << (log_n - log_s - log_next), scale ? *scale : one,
                            (int)(scale != nullptr));
     }
 }

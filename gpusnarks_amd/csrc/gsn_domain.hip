@@ -378,42 +378,21 @@ typename FieldInfo<FID>::Host value_r()
     return H::from_canonical(H::one().im_rep);  // one() holds R mod p
 }
 
-// the residue of a twiddle record
-inline void value_of(E753 &v, const TW753 &t)
-{
-    for (int l = 0; l < 24; ++l) {
-        uint64_t x = 0;
-        for (int d = 32 * l / 29; d < 26 && 29 * d < 32 * l + 32; ++d) {
-            const int at = 29 * d - 32 * l;
-            x |= at >= 0 ? (uint64_t)t.w[d] << at : (uint64_t)t.w[d] >> -at;
-        }
-        v.v[l] = (uint32_t)x;
-    }
-}
-
-// byte matrices of the residues of records
+// byte matrices of the residues of records, `count` in device memory or one;
+// on the null stream, asynchronous
 template <int FID>
-int build_matrices(DeviceBuffer &mat, const std::vector<TW753> &records)
+int build_matrices(void *mat, uint32_t count, const void *records, const TW753 &one = {})
 {
-    std::vector<E753> vals(records.size());
-    for (size_t i = 0; i < vals.size(); ++i)
-        value_of(vals[i], records[i]);
-    DeviceBuffer dv;
-    GSN_TRY(dv.alloc(vals.size() * sizeof(E753)));
-    GSN_TRY(hip_status(hipMemcpy(dv.ptr, vals.data(), vals.size() * sizeof(E753), hipMemcpyHostToDevice), "hipMemcpy"));
-    GSN_TRY(mat.alloc(vals.size() * MAT_BYTES));
-    launch_build_mat753_values<typename FieldInfo<FID>::Dev>((uint4 *)mat.ptr, (uint32_t)vals.size(),
-                                                             (const E753 *)dv.ptr, 0);
-    GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
-    return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
+    if constexpr (FID != GSN_FIELD_FP32)
+        launch_build_mat753_records<typename FieldInfo<FID>::Dev>((uint4 *)mat, count, (const TW753 *)records, one, 0);
+    return hip_status(hipGetLastError(), "matrix table launch");
 }
 
 struct CosetTables {
-    DeviceBuffer lo, hi;
-    DeviceBuffer mat;  // hi as byte matrices (coset_matrix), or empty
+    DeviceBuffer buf;  // hi and lo as records, then hi as byte matrices (coset_matrix) or nothing
+    const void *lo = nullptr, *hi = nullptr, *mat = nullptr;
     uint32_t h = 0;
-    bool matrix() const { return mat.ptr != nullptr; }
-    CosetArgs args() const { return CosetArgs{(const TW753 *)lo.ptr, mat.ptr, h}; }
+    CosetArgs args() const { return CosetArgs{(const TW753 *)lo, mat, h}; }
 };
 // Whether hi's products go to the matrix cores: 64 consecutive i share one
 // from 2^11 points (7.0 against 8.9 us there, 95 against 117 at 2^20).  These
@@ -447,35 +426,42 @@ int coset_tables(CosetTables **out, const typename FieldInfo<FID>::Host &g, unsi
         const H base = inverse ? g.mul_inv() : g;
         t->h = (log_n + 1) / 2;
         const size_t nlo = (size_t)1 << t->h, nhi = std::max<size_t>(1, ((size_t)1 << log_n) >> t->h);
-        std::vector<tw> lo(nlo), hi(nhi);
-        H acc = H::one();
-        for (size_t x = 0; x < nlo; ++x) {
-            lo[x] = record<FID>(acc);
-            acc *= base;
+        const size_t records = ((nlo + nhi) * sizeof(tw) + 255) & ~(size_t)255;
+        size_t matrices = coset_matrix<FID>(log_n) ? nhi * MAT_BYTES : 0;
+        if (g_coset_matrix_bytes + matrices > COSET_MATRIX_BYTES)
+            matrices = 0;
+        if (matrices && t->buf.alloc(records + matrices) == GSN_ERR_OUT_OF_MEMORY) {
+            matrices = 0;
+            t->buf = DeviceBuffer();
+            (void)hipGetLastError();
         }
-        const H step = acc;
-        acc = H::one();
-        for (size_t y = 0; y < nhi; ++y) {
-            hi[y] = record<FID>(acc);
-            acc *= step;
-        }
-        GSN_TRY(t->lo.alloc(nlo * sizeof(tw)));
-        GSN_TRY(t->hi.alloc(nhi * sizeof(tw)));
-        GSN_TRY(hip_status(hipMemcpy(t->lo.ptr, lo.data(), nlo * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
-        GSN_TRY(hip_status(hipMemcpy(t->hi.ptr, hi.data(), nhi * sizeof(tw), hipMemcpyHostToDevice), "hipMemcpy"));
-        if constexpr (FID != GSN_FIELD_FP32) {
-            const size_t bytes = nhi * MAT_BYTES;
-            if (coset_matrix<FID>(log_n) && g_coset_matrix_bytes + bytes <= COSET_MATRIX_BYTES) {
-                const int st = build_matrices<FID>(t->mat, hi);
-                if (st == GSN_ERR_OUT_OF_MEMORY) {
-                    t->mat = DeviceBuffer();
-                    (void)hipGetLastError();
-                } else {
-                    GSN_TRY(st);
-                    g_coset_matrix_bytes += bytes;
-                }
+        GSN_TRY(t->buf.alloc(records + matrices));
+        char *const at = (char *)t->buf.ptr;
+        t->hi = at;
+        t->lo = at + nhi * sizeof(tw);
+        std::vector<tw> rec(std::max(nlo, nhi));
+        const auto upload = [&](const H &factor, size_t count, const void *to) {
+            H acc = H::one();
+            for (size_t x = 0; x < count; ++x) {
+                rec[x] = record<FID>(acc);
+                acc *= factor;
             }
+            return hip_status(hipMemcpy((void *)to, rec.data(), count * sizeof(tw), hipMemcpyHostToDevice),
+                              "hipMemcpy");
+        };
+        // hi first, so that its matrices are built while the host forms lo
+        H step = base;
+        for (uint32_t i = 0; i < t->h; ++i)
+            step *= step;
+        GSN_TRY(upload(step, nhi, t->hi));
+        if (matrices) {
+            t->mat = at + records;
+            GSN_TRY(build_matrices<FID>(at + records, (uint32_t)nhi, t->hi));
         }
+        GSN_TRY(upload(base, nlo, t->lo));
+        if (matrices)
+            GSN_TRY(hip_status(hipStreamSynchronize(nullptr), "coset tables"));
+        g_coset_matrix_bytes += matrices;
         slot = std::move(t);
     }
     *out = slot.get();
@@ -504,14 +490,14 @@ int coset_t(void *out, const void *in, size_t n, const void *g_limbs, int invers
     CosetTables *t = nullptr;
     GSN_TRY(coset_tables<FID>(&t, g, log_n, inverse));
     if constexpr (FID != GSN_FIELD_FP32) {
-        if (t->matrix()) {
+        if (t->mat) {
             launch_coset753<F>((E753 *)out, (const E753 *)in, t->args(), n, st);
             return hip_status(hipGetLastError(), "coset launch");
         }
     }
     hipLaunchKernelGGL(ew_coset_kernel<F>, dim3(blocks_for(n)), dim3(256), 0, st, (typename F::elem_t *)out,
-                       (const typename F::elem_t *)in, (const typename F::tw_t *)t->lo.ptr,
-                       (const typename F::tw_t *)t->hi.ptr, t->h, n);
+                       (const typename F::elem_t *)in, (const typename F::tw_t *)t->lo,
+                       (const typename F::tw_t *)t->hi, t->h, n);
     return hip_status(hipGetLastError(), "coset launch");
 }
 
@@ -579,7 +565,7 @@ struct ExtPlan : PlanBase {
     PlanBase *half = nullptr;
     CosetTables *tab = nullptr;  // g^i (forward) or g^-i (inverse), i < m
     typename F::tw_t c;          // G (forward) or 1 / (1 - G) (inverse)
-    DeviceBuffer cmat;           // its matrix, where tab has them
+    DeviceBuffer cmat;           // its matrix, for use with tab's
     std::unique_ptr<BatchImpl> halves;  // both half transforms, fused
     const void *halves_in = nullptr;
     void *halves_out = nullptr;
@@ -612,7 +598,7 @@ struct ExtPlan : PlanBase {
     bool matrix_step(const void *in, void *out, size_t m, hipStream_t st)
     {
         if constexpr (FID != GSN_FIELD_FP32) {
-            if (tab->matrix()) {
+            if (tab->mat) {
                 launch_ext753<F>((E753 *)out, (const E753 *)in, tab->args(), cmat.ptr, m, inverse, st);
                 return true;
             }
@@ -629,12 +615,15 @@ struct ExtPlan : PlanBase {
         const H G = g.pow((uint64_t)1 << lm);
         if (G == H::one())
             return set_error(GSN_ERR_INVALID_ARGUMENT, "shift^(n/2) = 1: g*H would meet H");
-        GSN_TRY(create_plan(&half, FID, lm, nullptr, inv));
-        GSN_TRY(coset_tables<FID>(&tab, g, lm, inv));
         c = inv ? record<FID>((H::one() - G).mul_inv()) : record<FID>(G);
         if constexpr (FID != GSN_FIELD_FP32)
-            if (tab->matrix())
-                GSN_TRY(build_matrices<FID>(cmat, {c}));
+            if (coset_matrix<FID>(lm)) {
+                GSN_TRY(cmat.alloc(MAT_BYTES));
+                GSN_TRY(build_matrices<FID>(cmat.ptr, 1, nullptr, c));
+            }
+        GSN_TRY(create_plan(&half, FID, lm, nullptr, inv));
+        GSN_TRY(coset_tables<FID>(&tab, g, lm, inv));
+        GSN_TRY(hip_status(hipStreamSynchronize(nullptr), "matrix tables"));
         num_passes = half->num_passes + 1;  // the halves' passes are fused
         device_bytes = half->device_bytes;
         return GSN_OK;
@@ -645,7 +634,7 @@ struct ExtPlan : PlanBase {
         using E = typename F::elem_t;
         const size_t m = (size_t)1 << (log_n - 1);
         const dim3 grid(blocks_for(m)), block(256);
-        const auto *lo = (const typename F::tw_t *)tab->lo.ptr, *hi = (const typename F::tw_t *)tab->hi.ptr;
+        const auto *lo = (const typename F::tw_t *)tab->lo, *hi = (const typename F::tw_t *)tab->hi;
         if (!inverse) {
             GSN_TRY(take_injected_fault());
             if (!matrix_step(in, out, m, st))
@@ -702,8 +691,11 @@ struct MixedPlan : PlanBase {
     using TW = typename O::tw;
     uint32_t n1 = 0, a = 0, h = 0;
     MixRadices rad{};
-    DeviceBuffer T, lo, hi, ws, ws2, CS;  // T, lo, hi, CS: records of constants
-    DeviceBuffer mat;                     // the byte matrices of T, then of CS (matrix())
+    DeviceBuffer T, lo, hi, ws, ws2;  // T (the powers of w_{n1}, then the DFT constants), lo, hi: records
+    const TW *CS = nullptr;           // the DFT constants
+    // byte matrices: T's (matrix()), then those of the column passes (columns())
+    DeviceBuffer mat;
+    const void *fold1 = nullptr, *fold2 = nullptr;
     std::unique_ptr<BatchImpl> rows;
 
     static void put(std::vector<TW> &v, size_t i, const H &x) { v[i] = record<FID>(x); }
@@ -721,43 +713,45 @@ struct MixedPlan : PlanBase {
         uint32_t r1 = 0, r2 = 0;
         return matrix() && columns_split(a, r1, r2);
     }
-    DeviceBuffer fold1, fold2;
-    // byte matrices of the powers of wr, of order 2^a, for both passes
-    int build_columns(const H &wr)
+    // the matrices of T and, for both column passes, of the powers of wr, of
+    // order 2^a
+    int build_mats(const H &wr)
     {
         if constexpr (FID != GSN_FIELD_FP32) {
             using F = typename FieldInfo<FID>::Dev;
-            const uint32_t hb = (a + 1) / 2;
-            std::vector<TW> vlo((size_t)1 << hb);
-            std::vector<E753> vhi((size_t)1 << (a - hb));
-            H acc = H::one();
-            for (TW &t : vlo) {
-                t = record<FID>(acc);
-                acc = acc * wr;
-            }
-            const H step = acc;
-            acc = H::one();
-            for (E753 &v : vhi) {
-                acc.to_canonical(v.v);
-                acc = acc * step;
-            }
-            DeviceBuffer dlo, dhi;
-            GSN_TRY(dlo.alloc(vlo.size() * sizeof(TW)));
-            GSN_TRY(dhi.alloc(vhi.size() * sizeof(E753)));
-            GSN_TRY(hip_status(hipMemcpy(dlo.ptr, vlo.data(), vlo.size() * sizeof(TW), hipMemcpyHostToDevice),
-                               "hipMemcpy"));
-            GSN_TRY(hip_status(hipMemcpy(dhi.ptr, vhi.data(), vhi.size() * sizeof(E753), hipMemcpyHostToDevice),
-                               "hipMemcpy"));
+            const uint32_t e0 = n1 + MIX_CS_ELEMS;
             uint32_t r1 = 0, r2 = 0;
-            columns_split(a, r1, r2);
+            const bool cols = columns_split(a, r1, r2);
             const uint32_t e1 = (1u << r1) - 1u, e2 = ((1u << r2) - 1u) << r1;
-            GSN_TRY(fold1.alloc((size_t)e1 * MAT_BYTES));
-            GSN_TRY(fold2.alloc((size_t)e2 * MAT_BYTES));
-            launch_build_mat753<F>((uint4 *)fold1.ptr, e1, true, (const E753 *)dhi.ptr, (const TW753 *)dlo.ptr, hb, a,
-                                   0, 0, 0, false, nullptr, 0);
-            launch_build_mat753<F>((uint4 *)fold2.ptr, e2, true, (const E753 *)dhi.ptr, (const TW753 *)dlo.ptr, hb, a,
-                                   r1, 0, 0, false, nullptr, 0);
-            GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+            GSN_TRY(mat.alloc((size_t)(cols ? e0 + e1 + e2 : e0) * MAT_BYTES));
+            GSN_TRY(build_matrices<FID>(mat.ptr, e0, T.ptr));
+            DeviceBuffer roots;  // the records of wr^e, e < 2^hb, then the residues of its powers of order 2^(a - hb)
+            if (cols) {
+                fold1 = (const char *)mat.ptr + (size_t)e0 * MAT_BYTES;
+                fold2 = (const char *)fold1 + (size_t)e1 * MAT_BYTES;
+                const uint32_t hb = (a + 1) / 2;
+                const size_t nlo = (size_t)1 << hb, nhi = (size_t)1 << (a - hb);
+                std::vector<char> both(nlo * sizeof(TW) + nhi * sizeof(E753));
+                H acc = H::one();
+                for (size_t i = 0; i < nlo; ++i, acc = acc * wr) {
+                    const TW t = record<FID>(acc);
+                    std::memcpy(both.data() + i * sizeof(TW), &t, sizeof(TW));
+                }
+                const H step = acc;
+                acc = H::one();
+                for (size_t i = 0; i < nhi; ++i, acc = acc * step) {
+                    E753 v;
+                    acc.to_canonical(v.v);
+                    std::memcpy(both.data() + nlo * sizeof(TW) + i * sizeof(E753), &v, sizeof(E753));
+                }
+                GSN_TRY(roots.alloc(both.size()));
+                GSN_TRY(hip_status(hipMemcpy(roots.ptr, both.data(), both.size(), hipMemcpyHostToDevice), "hipMemcpy"));
+                const TW753 *dlo = (const TW753 *)roots.ptr;
+                const E753 *dhi = (const E753 *)(dlo + nlo);
+                launch_build_mat753<F>((uint4 *)fold1, e1, true, dhi, dlo, hb, a, 0, 0, 0, false, nullptr, 0);
+                launch_build_mat753<F>((uint4 *)fold2, e2, true, dhi, dlo, hb, a, r1, 0, 0, false, nullptr, 0);
+                GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+            }
             GSN_TRY(hip_status(hipStreamSynchronize(nullptr), "matrix tables"));
         }
         return GSN_OK;
@@ -779,14 +773,13 @@ struct MixedPlan : PlanBase {
         const H w = w2 * MI::root_odd().pow(MI::ODD_MAX / n1);
         const H base = inv ? w.mul_inv() : w;
         // T[e] = (base^n2)^e, e < n1
-        std::vector<TW> t(n1);
+        std::vector<TW> t(n1 + MIX_CS_ELEMS);
         const H w1 = base.pow(n2);
         H acc = H::one();
         for (uint32_t e = 0; e < n1; ++e, acc = acc * w1)
             put(t, e, acc);
         // symmetric DFT constants per radix q: u = w1^(n1/q), C[e] = (u^e +
         // u^-e)/2, S[e] = (u^e - u^-e)/2
-        std::vector<TW> cs(MIX_CS_ELEMS);
         const H half = H(2u).mul_inv();
         for (uint32_t q : {3u, 5u, 7u}) {
             if (n1 % q)
@@ -794,8 +787,8 @@ struct MixedPlan : PlanBase {
             const H u = w1.pow(n1 / q), ui = u.mul_inv();
             H up = H::one(), un = H::one();
             for (uint32_t e = 0; e < q; ++e, up = up * u, un = un * ui) {
-                put(cs, mix_cs_offset(q) + e, (up + un) * half);
-                put(cs, mix_cs_offset(q) + q + e, (up - un) * half);
+                put(t, n1 + mix_cs_offset(q) + e, (up + un) * half);
+                put(t, n1 + mix_cs_offset(q) + q + e, (up - un) * half);
             }
         }
         // base^e = lo[e mod 2^h] hi[e >> h] (hi scaled by n1^-1 for the
@@ -810,30 +803,21 @@ struct MixedPlan : PlanBase {
         H hacc = inv ? H(columns() ? (uint32_t)n : n1).mul_inv() : H::one();
         for (size_t y = 0; y < nhi; ++y, hacc = hacc * acc)
             put(vhi, y, hacc);
-        GSN_TRY(T.alloc(n1 * sizeof(TW)));
+        GSN_TRY(T.alloc(t.size() * sizeof(TW)));
+        CS = (const TW *)T.ptr + n1;
         GSN_TRY(lo.alloc(nlo * sizeof(TW)));
         GSN_TRY(hi.alloc(nhi * sizeof(TW)));
         GSN_TRY(ws.alloc(n * sizeof(E)));
         if (rad.count > 1)
             GSN_TRY(ws2.alloc(n * sizeof(E)));
-        GSN_TRY(CS.alloc(MIX_CS_ELEMS * sizeof(TW)));
-        GSN_TRY(hip_status(hipMemcpy(CS.ptr, cs.data(), MIX_CS_ELEMS * sizeof(TW), hipMemcpyHostToDevice),
-                           "hipMemcpy"));
-        GSN_TRY(hip_status(hipMemcpy(T.ptr, t.data(), n1 * sizeof(TW), hipMemcpyHostToDevice), "hipMemcpy"));
+        GSN_TRY(hip_status(hipMemcpy(T.ptr, t.data(), t.size() * sizeof(TW), hipMemcpyHostToDevice), "hipMemcpy"));
         GSN_TRY(hip_status(hipMemcpy(lo.ptr, vlo.data(), nlo * sizeof(TW), hipMemcpyHostToDevice), "hipMemcpy"));
         GSN_TRY(hip_status(hipMemcpy(hi.ptr, vhi.data(), nhi * sizeof(TW), hipMemcpyHostToDevice), "hipMemcpy"));
-        if constexpr (FID != GSN_FIELD_FP32) {
-            if (matrix()) {
-                std::vector<TW753> both(t.begin(), t.end());
-                both.insert(both.end(), cs.begin(), cs.end());
-                GSN_TRY(build_matrices<FID>(mat, both));
-            }
-        }
+        if (matrix())
+            GSN_TRY(build_mats(base.pow(n1)));
         num_passes = 2;
         device_bytes = mat.bytes + (n1 + nlo + nhi + MIX_CS_ELEMS) * sizeof(TW) + (rad.count > 1 ? 2 : 1) * n * sizeof(E);
         if (columns()) {
-            GSN_TRY(build_columns(base.pow(n1)));
-            device_bytes += fold1.bytes + fold2.bytes;
             num_passes += 2;
         } else if (a > 0) {
             // the rows: radix-2 transforms over w^n1 (a primitive 2^a-th root)
@@ -874,13 +858,13 @@ struct MixedPlan : PlanBase {
                 }
             }
             if (q == 7)
-                launch_mixed_pass<O, 7>(last, dst, src, n1, a, L, (const TW *)T.ptr, (const TW *)CS.ptr,
+                launch_mixed_pass<O, 7>(last, dst, src, n1, a, L, (const TW *)T.ptr, CS,
                                         (const TW *)lo.ptr, (const TW *)hi.ptr, h, st);
             else if (q == 5)
-                launch_mixed_pass<O, 5>(last, dst, src, n1, a, L, (const TW *)T.ptr, (const TW *)CS.ptr,
+                launch_mixed_pass<O, 5>(last, dst, src, n1, a, L, (const TW *)T.ptr, CS,
                                         (const TW *)lo.ptr, (const TW *)hi.ptr, h, st);
             else
-                launch_mixed_pass<O, 3>(last, dst, src, n1, a, L, (const TW *)T.ptr, (const TW *)CS.ptr,
+                launch_mixed_pass<O, 3>(last, dst, src, n1, a, L, (const TW *)T.ptr, CS,
                                         (const TW *)lo.ptr, (const TW *)hi.ptr, h, st);
             src = dst;
             L *= q;
@@ -894,7 +878,7 @@ struct MixedPlan : PlanBase {
                                   (const TW753 *)lo.ptr, (const TW753 *)hi.ptr, h};
                 launch_mixed_twist<typename FieldInfo<FID>::Dev>(p, st);
                 launch_columns753<typename FieldInfo<FID>::Dev>((const E753 *)out, (E753 *)out, (E753 *)ws.ptr, a, n1,
-                                                                fold1.ptr, fold2.ptr, st);
+                                                                fold1, fold2, st);
                 return hip_status(hipGetLastError(), "mixed-radix columns launch");
             }
         }

@@ -454,12 +454,11 @@ int PlanImpl<GSN_FIELD_FP32>::build_tables(const fields::Fp32 &w, size_t n)
 template <class Plan, class H, class F, class P>
 static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
 {
-    // every record is w_n^e = hi[e >> h] * lo[e & (2^h - 1)] for e < n/2
-    // (e < n for matrix passes),
+    // every record is w_n^e = hi[e >> h] * lo[e & (2^h - 1)] for e < n/2,
     // computed on the device from hi (canonical residues) and lo (records)
     const bool mat = plan.cfg[0].kind != 0;
     const unsigned h = (log_n + 1) / 2;
-    const size_t nlo = (size_t)1 << h, nhi = std::max<size_t>(1, (mat ? n : n / 2) >> h);
+    const size_t nlo = (size_t)1 << h, nhi = std::max<size_t>(1, (n / 2) >> h);
     std::vector<TW753> lo(nlo);
     std::vector<E753> hi(nhi);
     H acc = H::one();
@@ -473,72 +472,80 @@ static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
         acc.to_canonical(hi[y].v);  // w^(y 2^h)
         acc *= step;
     }
-    DeviceBuffer dlo, dhi;
-    GSN_TRY(dlo.alloc(nlo * sizeof(TW753)));
-    GSN_TRY(dhi.alloc(nhi * sizeof(E753)));
-    GSN_TRY(hip_status(hipMemcpy(dlo.ptr, lo.data(), nlo * sizeof(TW753), hipMemcpyHostToDevice), "hipMemcpy"));
-    GSN_TRY(hip_status(hipMemcpy(dhi.ptr, hi.data(), nhi * sizeof(E753), hipMemcpyHostToDevice), "hipMemcpy"));
+    std::vector<char> both(nlo * sizeof(TW753) + nhi * sizeof(E753));
+    std::memcpy(both.data(), lo.data(), nlo * sizeof(TW753));
+    std::memcpy(both.data() + nlo * sizeof(TW753), hi.data(), nhi * sizeof(E753));
+    DeviceBuffer roots;
+    GSN_TRY(roots.alloc(both.size()));
+    GSN_TRY(hip_status(hipMemcpy(roots.ptr, both.data(), both.size(), hipMemcpyHostToDevice), "hipMemcpy"));
+    const TW753 *const dlo = (const TW753 *)roots.ptr;
+    const E753 *const dhi = (const E753 *)((const char *)roots.ptr + nlo * sizeof(TW753));
     const size_t P_ = plan.cfg.size();
     plan.step_tabs.resize(P_);
     plan.step_nrec.assign(P_, 0);
     unsigned log_ns = 0;
     if (mat) {
-        plan.mat_tabs.resize(3 * P_);
+        const bool dense = plan.cfg[0].kind == MAT_DENSE;
+        const auto r = [&](size_t i) { return (unsigned)plan.cfg[i].log_r; };
+        // a pass's matrices are those of the first one with the same radix and
+        // (not dense, from the second pass on) the same one before it
         plan.mat_share.resize(P_);
-        const auto build = [&](DeviceBuffer &b, size_t entries, bool fold, unsigned log_y, uint64_t mul, uint64_t add,
-                               bool pair, const TW753 *scale) {
-            GSN_TRY(b.alloc(entries * MAT_BYTES));
-            launch_build_mat753<F>((uint4 *)b.ptr, (uint32_t)entries, fold, (const E753 *)dhi.ptr,
-                                   (const TW753 *)dlo.ptr, h, log_n, log_y, mul, add, pair, scale, 0);
-            return hip_status(hipGetLastError(), "matrix table launch");
-        };
-        if (plan.cfg[0].kind == MAT_DENSE) {
-            for (size_t i = 0; i < P_; ++i) {
-                const unsigned r = (unsigned)plan.cfg[i].log_r;
-                size_t own = 0;
-                while (plan.cfg[own].log_r != (int)r)
-                    ++own;
-                plan.mat_share[i] = (int)own;
-                log_ns += r;
-                DeviceBuffer &mat = plan.mat_tabs[3 * i], &rec = plan.mat_tabs[3 * i + 1];
-                if (own == i)
-                    GSN_TRY(mat.alloc((size_t)MAT_BYTES << r));
-                unsigned next = 0;
-                if (i + 1 < P_) {
-                    next = (unsigned)plan.cfg[i + 1].log_r;
-                    GSN_TRY(rec.alloc(sizeof(TW753) << (log_ns + next)));
-                }
-                // n^-1 on the first pass's records
-                launch_build_dense753<F>((uint4 *)mat.ptr, r, (TW753 *)rec.ptr, log_ns, next, (const E753 *)dhi.ptr,
-                                         (const TW753 *)dlo.ptr, h, log_n,
-                                         i == 0 && plan.inverse ? &plan.scale : nullptr, 0);
-                GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
-            }
-            return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
-        }
-        const unsigned rp = (unsigned)plan.cfg[P_ - 1].log_r;
         for (size_t i = 0; i < P_; ++i) {
-            const unsigned r = (unsigned)plan.cfg[i].log_r, g = i ? (unsigned)plan.cfg[i - 1].log_r : 0u;
-            size_t own = i;
-            for (size_t k = 1; k < i; ++k)
-                if (plan.cfg[k].log_r == (int)r && plan.cfg[k - 1].log_r == (int)g)
-                    own = std::min(own, k);
+            size_t own = dense || i == 0 ? 0 : 1;
+            while (r(own) != r(i) || (!dense && i > 0 && r(own - 1) != r(i - 1)))
+                ++own;
             plan.mat_share[i] = (int)own;
-            if (own == i)
-                GSN_TRY(build(plan.mat_tabs[3 * i], (((size_t)1 << r) - 1) << g, true, g, 0, 0, false, nullptr));
-            if (i > 0 && i < P_ - 1) {
-                // column factors w_n^(jP k(i-1) N1..N(i-2)); n^-1 on the first
-                GSN_TRY(build(plan.mat_tabs[3 * i + 1], (size_t)1 << (g + rp), false, rp,
-                              (uint64_t)1 << (log_ns - g), 0, false, i == 1 && plan.inverse ? &plan.scale : nullptr));
-                if (i + 2 < P_) {  // the pair (1, 3)
-                    const unsigned r3 = (unsigned)plan.cfg[2].log_r;
-                    GSN_TRY(build(plan.mat_tabs[3 * i + 2], (size_t)2 << (g + r3), false, r3, (uint64_t)1 << rp,
-                                  n >> (g + 1), true, nullptr));
-                }
-            }
-            log_ns += r;
         }
-        GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+        const auto owns = [&](size_t i) { return plan.mat_share[i] == (int)i; };
+        const auto between = [&](size_t i) { return i > 0 && i + 1 < P_; };
+        // entries of table k of pass i: folded, column and fixed matrices, or
+        // (dense) matrices and records
+        const auto entries = [&](size_t i, int k, unsigned before) -> size_t {
+            const unsigned g = i ? r(i - 1) : 0u;
+            if (dense)
+                return k == 0 ? (owns(i) ? (size_t)1 << r(i) : 0)
+                              : k == 1 && i + 1 < P_ ? (size_t)1 << (before + r(i) + r(i + 1)) : 0;
+            switch (k) {
+            case 0: return owns(i) ? (((size_t)1 << r(i)) - 1) << g : 0;
+            case 1: return between(i) ? (size_t)1 << (g + r(P_ - 1)) : 0;
+            default: return between(i) && i + 2 < P_ ? (size_t)2 << (g + r(2)) : 0;
+            }
+        };
+        std::vector<size_t> at(3 * P_ + 1, 0);
+        for (size_t i = 0; i < P_; log_ns += r(i), ++i)
+            for (int k = 0; k < 3; ++k) {
+                const size_t bytes = entries(i, k, log_ns) * (dense && k == 1 ? sizeof(TW753) : (size_t)MAT_BYTES);
+                at[3 * i + k + 1] = at[3 * i + k] + ((bytes + 255) & ~(size_t)255);
+            }
+        GSN_TRY(plan.mat_buf.alloc(at.back()));
+        plan.mat_tabs.resize(3 * P_);
+        for (size_t x = 0; x < 3 * P_; ++x)
+            plan.mat_tabs[x] = at[x + 1] > at[x] ? (char *)plan.mat_buf.ptr + at[x] : nullptr;
+        log_ns = 0;
+        for (size_t i = 0; i < P_; log_ns += r(i), ++i) {
+            void *const *t = &plan.mat_tabs[3 * i];
+            const unsigned g = i ? r(i - 1) : 0u;
+            if (dense) {
+                // n^-1 on the first pass's records
+                launch_build_dense753<F>((uint4 *)t[0], r(i), (TW753 *)t[1], log_ns + r(i), t[1] ? r(i + 1) : 0u, dhi,
+                                         dlo, h, log_n, i == 0 && plan.inverse ? &plan.scale : nullptr, 0);
+            } else {
+                const auto build = [&](int k, bool fold, unsigned log_y, uint64_t mul, uint64_t add, bool pair,
+                                       const TW753 *scale) {
+                    if (t[k])
+                        launch_build_mat753<F>((uint4 *)t[k], (uint32_t)entries(i, k, log_ns), fold, dhi, dlo, h,
+                                               log_n, log_y, mul, add, pair, scale, 0);
+                };
+                build(0, true, g, 0, 0, false, nullptr);
+                // column factors w_n^(jP k(i-1) N1..N(i-2)); n^-1 on the first
+                build(1, false, r(P_ - 1), (uint64_t)1 << (log_ns - g), 0, false,
+                      i == 1 && plan.inverse ? &plan.scale : nullptr);
+                // the pair (1, 3)
+                if (t[2])
+                    build(2, false, r(2), (uint64_t)1 << r(P_ - 1), n >> (g + 1), true, nullptr);
+            }
+            GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+        }
         return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
     }
     for (size_t i = 0; i < P_; ++i) {
@@ -550,8 +557,8 @@ static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
         // the inverse's n^-1 rides on the last pass's step-0 records when
         // there is more than one pass (PASS_SCALE_IN)
         const bool scale0 = plan.inverse && P_ >= 2 && i == P_ - 1;
-        launch_build_steps753<F>((uint4 *)plan.step_tabs[i].ptr, nrec, (const E753 *)dhi.ptr, (const TW753 *)dlo.ptr,
-                                 h, log_n, log_ns, lr, plan.scale, scale0, 0);
+        launch_build_steps753<F>((uint4 *)plan.step_tabs[i].ptr, nrec, dhi, dlo, h, log_n, log_ns, lr, plan.scale,
+                                 scale0, 0);
         GSN_TRY(hip_status(hipGetLastError(), "build_steps753 launch"));
         log_ns += lr;
     }

@@ -770,26 +770,44 @@ __global__ __launch_bounds__(1 << (LOG_R + LOG_W - 2)) __attribute__((amdgpu_wav
     MatTile<F, KIND, LOG_R, LOG_W>(args, lds).run();
 }
 
-// w_n^e = hi[e >> h] * lo[e mod 2^h], canonical
+// w_n^e for e < n = 2^log_n, canonical: hi[e >> h] lo[e mod 2^h] for e < n/2,
+// and its negative past that
 template <class F>
-__device__ __forceinline__ E753 root_power(const E753 *hi, const TW753 *lo, uint32_t h, size_t e)
+__device__ __forceinline__ E753 root_power(const E753 *hi, const TW753 *lo, uint32_t h, uint32_t log_n, size_t e)
 {
-    return F::canon(F::mul(hi[e >> h], lo[e & (((size_t)1 << h) - 1u)]));
-}
-
-// The byte matrix of w: thread k < 96 forms column c_k, centred, as signed
-// digits in img.
-template <class F>
-__device__ __forceinline__ void matrix_image(uint8_t *img, const E753 &value, uint32_t k)
-{
-    using P = typename F::params;
-    const TW753 w = F::make_tw(value);
-    if (k < 96) {
-        E753 y;
+    const size_t half = (size_t)1 << (log_n - 1), x = e & (half - 1);
+    E753 v = F::canon(F::mul(hi[x >> h], F::load_tw(lo, x & (((size_t)1 << h) - 1u))));
+    if (e >= half) {
+        unsigned b = 0;
 #pragma unroll
         for (int l = 0; l < 24; ++l)
-            y.v[l] = (k >> 2) == (uint32_t)l ? 1u << (8 * (k & 3)) : 0u;
-        E753 v = F::canon(F::mul(y, w));
+            v.v[l] = __builtin_subc(F::params::MOD[l], v.v[l], b, &b);
+    }
+    return v;
+}
+
+// Byte matrices of the residues value(i), i < entries: a wavefront forms five,
+// 12 lanes each, a lane the columns 8 t .. 8 t + 7: the first as a product,
+// each next one as 256 times the one before it, centred and written as signed
+// digits.  A plan's thousands of matrices would otherwise be thousands of
+// products (a column each: 250 us for 4096, with the residues' own products,
+// the same for a whole block, on the scalar unit).
+constexpr uint32_t MATS_PER_WAVE = 5;
+template <class F, class V>
+__device__ __forceinline__ void write_matrices(uint4 *out, uint32_t entries, V value)
+{
+    using P = typename F::params;
+    __shared__ __align__(16) uint8_t img[MATS_PER_WAVE * MAT_BYTES];
+    const uint32_t first = blockIdx.x * MATS_PER_WAVE, group = threadIdx.x / 12;
+    const uint32_t t = threadIdx.x - 12 * group, m = min(group, MATS_PER_WAVE - 1);  // (four lanes repeat the last's)
+    const TW753 w = F::make_tw(value(min(first + m, entries - 1)));
+    E753 v;
+#pragma unroll
+    for (int l = 0; l < 24; ++l)
+        v.v[l] = (uint32_t)l == 2 * t ? 1u : 0u;
+    v = F::canon(F::mul(v, w));
+#pragma unroll 1
+    for (uint32_t k = 8 * t;;) {
         // centre: v - p when v > p/2 (compare the top limbs; either choice is
         // right to within 2^-16 p)
         unsigned b = 0;
@@ -804,45 +822,53 @@ __device__ __forceinline__ void matrix_image(uint8_t *img, const E753 &value, ui
             const uint32_t x = __builtin_addc(neg ? d.v[l] : v.v[l], Mat753<P>::K80, c, &c) ^ Mat753<P>::K80;
 #pragma unroll
             for (int byte = 0; byte < 4; ++byte) {
-                const uint32_t m = 4 * l + byte;
-                img[((m >> 5) * 3 + (k >> 5)) * 1024 + ((m & 31) + 32 * ((k & 31) >> 4)) * 16 + (k & 15)] =
-                    (uint8_t)(x >> (8 * byte));
+                const uint32_t r = 4 * l + byte;
+                img[m * MAT_BYTES + ((r >> 5) * 3 + (k >> 5)) * 1024 + ((r & 31) + 32 * ((k & 31) >> 4)) * 16 +
+                    (k & 15)] = (uint8_t)(x >> (8 * byte));
             }
         }
+        if ((++k & 7) == 0)
+            break;
+#pragma unroll
+        for (int l = 23; l > 0; --l)
+            v.v[l] = __builtin_amdgcn_alignbit(v.v[l], v.v[l - 1], 24);
+        v.v[0] <<= 8;
+        v = F::canon(v);
     }
+    __syncthreads();
+    const uint32_t quads = min(MATS_PER_WAVE, entries - first) * (MAT_BYTES / 16);
+    for (uint32_t q = threadIdx.x; q < quads; q += 64)
+        out[(size_t)first * (MAT_BYTES / 16) + q] = reinterpret_cast<const uint4 *>(img)[q];
 }
 
-// Matrices, a block per entry i.  FOLD: the twiddles of a pass's steps,
-// entry ((2^s - 1) << log_y) + (g << s) + kk being w_{G 2^(s+1)}^(g + G kk),
+// Matrices of entries i.  FOLD: the twiddles of a pass's steps, entry
+// ((2^s - 1) << log_y) + (g << s) + kk being w_{G 2^(s+1)}^(g + G kk),
 // G = 2^log_y.  Else entry x 2^log_y + y is w_n^(x y mul), times *scale if
 // use_scale; with pair, entries 2 (x 2^log_y + y) and the one after it are
 // that and its product with w_n^(x add).
 template <class F, bool FOLD>
-__global__ __launch_bounds__(128) void build_mat753_kernel(uint4 *out, const E753 *hi, const TW753 *lo, uint32_t h,
-                                                          uint32_t log_n, uint32_t log_y, uint64_t mul, uint64_t add,
-                                                          int pair, TW753 scale, int use_scale)
+__global__ __launch_bounds__(64) void build_mat753_kernel(uint4 *out, uint32_t entries, const E753 *hi,
+                                                         const TW753 *lo, uint32_t h, uint32_t log_n, uint32_t log_y,
+                                                         uint64_t mul, uint64_t add, int pair, TW753 scale,
+                                                         int use_scale)
 {
-    __shared__ __align__(16) uint8_t img[MAT_BYTES];
-    const uint32_t i = blockIdx.x, k = threadIdx.x;
-    size_t e;
-    if (FOLD) {
-        const uint32_t s = 31u - (uint32_t)__builtin_clz((i >> log_y) + 1u);
-        const uint32_t rest = i - (((1u << s) - 1u) << log_y);
-        const uint32_t g = rest >> s, kk = rest & ((1u << s) - 1u);
-        e = ((size_t)g + ((size_t)kk << log_y)) << (log_n - log_y - s - 1u);
-    } else {
-        const uint32_t z = pair ? i >> 1 : i;
-        const size_t x = z >> log_y, y = z & ((1u << log_y) - 1u);
-        e = x * y * mul + (pair && (i & 1) ? x * add : 0);
-    }
-    E753 v = root_power<F>(hi, lo, h, e);
-    if (use_scale)
-        v = F::canon(F::mul(v, scale));
-    matrix_image<F>(img, v, k);
-    __syncthreads();
-    for (uint32_t q = k; q < MAT_BYTES / 16; q += 128)
-        out[(size_t)i * (MAT_BYTES / 16) + q] = reinterpret_cast<const uint4 *>(img)[q];
+    write_matrices<F>(out, entries, [&](uint32_t i) {
+        size_t e;
+        if (FOLD) {
+            const uint32_t s = 31u - (uint32_t)__builtin_clz((i >> log_y) + 1u);
+            const uint32_t rest = i - (((1u << s) - 1u) << log_y);
+            const uint32_t g = rest >> s, kk = rest & ((1u << s) - 1u);
+            e = ((size_t)g + ((size_t)kk << log_y)) << (log_n - log_y - s - 1u);
+        } else {
+            const uint32_t z = pair ? i >> 1 : i;
+            const size_t x = z >> log_y, y = z & ((1u << log_y) - 1u);
+            e = x * y * mul + (pair && (i & 1) ? x * add : 0);
+        }
+        const E753 v = root_power<F>(hi, lo, h, log_n, e);
+        return use_scale ? F::canon(F::mul(v, scale)) : v;
+    });
 }
+constexpr uint32_t mat_blocks(uint32_t entries) { return (entries + MATS_PER_WAVE - 1) / MATS_PER_WAVE; }
 
 // tiles of 32 columns; 2^4 rows only in MAT_MID (matrix_passes uses no others)
 #define GSN_MAT753_CASE(F, K, R)                                                                                   \
@@ -882,11 +908,12 @@ __global__ __launch_bounds__(128) void build_mat753_kernel(uint4 *out, const E75
     {                                                                                                                 \
         const TW753 one{};                                                                                            \
         if (fold)                                                                                                     \
-            hipLaunchKernelGGL((build_mat753_kernel<F, true>), dim3(entries), dim3(128), 0, st, out, hi, lo, h,       \
-                               log_n, log_y, mul, add, 0, one, 0);                                                    \
+            hipLaunchKernelGGL((build_mat753_kernel<F, true>), dim3(mat_blocks(entries)), dim3(64), 0, st, out,       \
+                               entries, hi, lo, h, log_n, log_y, mul, add, 0, one, 0);                                \
         else                                                                                                          \
-            hipLaunchKernelGGL((build_mat753_kernel<F, false>), dim3(entries), dim3(128), 0, st, out, hi, lo, h,      \
-                               log_n, log_y, mul, add, (int)pair, scale ? *scale : one, (int)(scale != nullptr));     \
+            hipLaunchKernelGGL((build_mat753_kernel<F, false>), dim3(mat_blocks(entries)), dim3(64), 0, st, out,      \
+                               entries, hi, lo, h, log_n, log_y, mul, add, (int)pair, scale ? *scale : one,           \
+                               (int)(scale != nullptr));                                                              \
     }
 
 }  // namespace gsn

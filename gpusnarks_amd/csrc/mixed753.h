@@ -28,8 +28,10 @@ void launch_mixed_mat(const MixedPass &a, uint32_t q, bool last, hipStream_t str
 // positions.
 template <class F>
 void launch_mixed_twist(const MixedPass &a, hipStream_t stream);
-// The matrices of `count` canonical residues.
+// The matrices of the residues of `count` records in device memory or (null)
+// of `one`.
 template <class F>
-void launch_build_mat753_values(uint4 *out, uint32_t count, const E753 *values, hipStream_t stream);
+void launch_build_mat753_records(uint4 *out, uint32_t count, const TW753 *records, const TW753 &one,
+                                 hipStream_t stream);
 
 }  // namespace gsn

@@ -276,15 +276,21 @@ __global__ __launch_bounds__(256) void mixed_twist_kernel(MixedPass a)
                  twist<F>(F::load(a.src, ((size_t)pos << a.log_n2) + j2), a, (uint64_t)j2 * pos));
 }
 
-// matrices of given residues, a block each
+// matrices of the residues of records, or (null) of one
 template <class F>
-__global__ __launch_bounds__(128) void build_mat753_values_kernel(uint4 *out, const E753 *values)
+__global__ __launch_bounds__(64) void build_mat753_records_kernel(uint4 *out, uint32_t entries, const TW753 *records,
+                                                                 TW753 one)
 {
-    __shared__ __align__(16) uint8_t img[MAT_BYTES];
-    matrix_image<F>(img, values[blockIdx.x], threadIdx.x);
-    __syncthreads();
-    for (uint32_t q = threadIdx.x; q < MAT_BYTES / 16; q += 128)
-        out[(size_t)blockIdx.x * (MAT_BYTES / 16) + q] = reinterpret_cast<const uint4 *>(img)[q];
+    write_matrices<F>(out, entries, [&](uint32_t i) {
+        const TW753 r = records ? F::load_tw(records, i) : one;
+        uint32_t d[27];
+#pragma unroll
+        for (int l = 0; l < 27; ++l)
+            d[l] = l < 26 ? r.w[l] : 0u;
+        E753 v;
+        F::from29(v.v, d);
+        return v;
+    });
 }
 
 template <class F, int Q>
@@ -317,16 +323,17 @@ void launch_mixed_twist(const MixedPass &a, hipStream_t st)
     hipLaunchKernelGGL(mixed_twist_kernel<F>, dim3(((a.n1 + 3) / 4) << (a.log_n2 - 6)), dim3(256), 0, st, a);
 }
 template <class F>
-void launch_build_mat753_values(uint4 *out, uint32_t count, const E753 *values, hipStream_t st)
+void launch_build_mat753_records(uint4 *out, uint32_t count, const TW753 *records, const TW753 &one, hipStream_t st)
 {
-    hipLaunchKernelGGL(build_mat753_values_kernel<F>, dim3(count), dim3(128), 0, st, out, values);
+    hipLaunchKernelGGL(build_mat753_records_kernel<F>, dim3(mat_blocks(count)), dim3(64), 0, st, out, count, records,
+                       one);
 }
 
 template void launch_mixed_mat<FMnt4>(const MixedPass &, uint32_t, bool, hipStream_t);
 template void launch_mixed_mat<FMnt6>(const MixedPass &, uint32_t, bool, hipStream_t);
 template void launch_mixed_twist<FMnt4>(const MixedPass &, hipStream_t);
 template void launch_mixed_twist<FMnt6>(const MixedPass &, hipStream_t);
-template void launch_build_mat753_values<FMnt4>(uint4 *, uint32_t, const E753 *, hipStream_t);
-template void launch_build_mat753_values<FMnt6>(uint4 *, uint32_t, const E753 *, hipStream_t);
+template void launch_build_mat753_records<FMnt4>(uint4 *, uint32_t, const TW753 *, const TW753 &, hipStream_t);
+template void launch_build_mat753_records<FMnt6>(uint4 *, uint32_t, const TW753 *, const TW753 &, hipStream_t);
 
 }  // namespace gsn

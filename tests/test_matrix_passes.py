@@ -248,3 +248,21 @@ def test_addresses_and_entries_of_every_schedule(log_n):
         assert kap.min() >= 0 and kap.max() < 1 << log_g
         assert (((1 << s) - 1) << log_g) + (kap.max() << s) + (1 << s) - 1 < ((1 << r) - 1) << log_g
         log_ns += r
+
+
+@pytest.mark.parametrize("field", FIELDS)
+def test_columns_in_runs_of_eight(field):
+    """write_matrices: twelve lanes with eight columns each, the first one
+    256^(8 t) w mod p and every next one 256 times the one before it, which
+    canon takes below 2^761."""
+    p = g.MODULI[field]
+    rng = random.Random(field + 200)
+    for w in [0, 1, p - 1, p // 2] + [rng.randrange(p) for _ in range(4)]:
+        got = []
+        for t in range(12):
+            c = (w << (64 * t)) % p
+            for k in range(8):
+                got.append(c - p if (c >> 736) > (p >> 736) // 2 else c)
+                assert c << 8 < 1 << 761
+                c = (c << 8) % p
+        assert got == columns(w, p)
