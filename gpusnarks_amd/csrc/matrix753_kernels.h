@@ -25,9 +25,12 @@
 // so that the bytes of x^, each with its top bit flipped, are exactly the
 // signed digits of x; sums and differences x0 +- t keep the offset.
 //
-// Bounds.  A product is below B = 6144 p.  x0 is reduced to about p/2 at
-// every second step, so values stay below 2 B + 6 p < 2^766.5, inside the
-// digits' range of 127/255 2^768.
+// Bounds.  A product is below B = 6144 (1 + 2^-15) p.  x0 is reduced to about
+// p/2 at every second step, so values stay below 2 B + 6 p, but for two places
+// where a third product comes before the next reduction: step 1 of MAT_MID2
+// (both halves of whose step 0 are products) and step 0 of COL_LAST (which
+// reads what COL_FIRST left, up to 2 B + p).  VALUE_MAX p = 3 B + p is inside
+// the digits' range, 127/255 2^768, by 0.1%.
 #pragma once
 
 #include <type_traits>
@@ -53,9 +56,13 @@ struct Mat753 {
     // 2^768, which row 0 makes up for.
     static constexpr int BIAS = (1 << 22) - (1 << 14);
     static constexpr uint32_t BIAS_ROW0 = 1u << 14;
-    // a multiple of p above the bound of any value: x + LIFT p is positive
-    // and below 2^768
-    static constexpr uint32_t LIFT = 12400u;
+    static constexpr uint32_t VALUE_MAX = 18434u;
+    static_assert((uint64_t)VALUE_MAX * (P::MOD[23] + 1ull) <= 0x7F7F7F7Full, "values are sums of signed byte digits");
+    // a multiple of p above what a last pass or a single product leaves, 2 B + p
+    // at most: x + LIFT p is positive and below 2^768
+    static constexpr uint32_t LIFTED_MAX = 12290u, LIFT = 12400u;
+    static_assert(LIFT > LIFTED_MAX && (uint64_t)(LIFT + LIFTED_MAX) * (P::MOD[23] + 1ull) < 1ull << 32,
+                  "lifted values are positive and below 2^768");
 
     static constexpr W24 lift_offset()  // LIFT p - 0x8080..80 mod 2^768
     {
@@ -457,8 +464,9 @@ struct MatTile {
                                                            (int)entry, i * (64 / GROUPS)) * MAT_BYTES);
         mat753_mul<P, GROUPS, BUTTERFLY>(b0, b1, m, bias, x0, v);
     }
-    // the steps that reduce x0 first: inputs are below 2 B in MAT_MID, below
-    // B in MAT_LAST and below 6 p after the two plain steps of MAT_FIRST
+    // the steps that reduce x0 first: inputs are below 2 B + 6 p in MAT_MID,
+    // below B in MAT_LAST, below 2 B + p in COL_LAST and below 6 p after the two
+    // plain steps of MAT_FIRST
     static constexpr bool reduces(int s) { return MID ? s % 2 == 0 : ENDS ? s % 2 == 1 : s % 2 == 1 && s >= 3; }
 
     // step s on elements lo (bit clear) and up; kk = low K bits of jj plus

@@ -266,3 +266,64 @@ def test_columns_in_runs_of_eight(field):
                 assert c << 8 < 1 << 761
                 c = (c << 8) % p
         assert got == columns(w, p)
+
+
+VALUE_MAX, LIFTED_MAX = 18434, 12290  # in units of p
+DIGITS_MAX = int("7f" * 96, 16)
+
+
+def magnitudes(kind, r, start):
+    """Largest value met in a pass of 2^r rows whose inputs are below `start`,
+    and what it leaves, in units of p."""
+    B = 6144 * (1 + 2.0 ** -15)
+    v = seen = start
+    for s in range(r):
+        if kind == "first" and s < 2:  # sums, and at step 1 products by w_4
+            v = 2 * v if s == 0 else max(2 * v, v + B)
+        elif kind == "mid2" and s == 0:  # both halves are products
+            v = 2 * B
+        else:
+            reduced = {"first": s % 2 == 1, "mid": s % 2 == 0, "mid2": s % 2 == 0}.get(kind, s % 2 == 1)
+            v = (0.51 if reduced else v) + B
+        seen = max(seen, v)
+    return seen, v
+
+
+def test_values_of_every_schedule_stay_in_range():
+    """The bounds that the passes are built on, followed through every schedule
+    and every pair of column passes; 3 B is reached in MAT_MID2 and COL_LAST."""
+    B = 6144 * (1 + 2.0 ** -15)
+    most = {}
+    for radices in SCHEDULES.values():
+        num, v = len(radices), 1.0
+        for i, r in enumerate(radices):
+            kind = "first" if i == 0 else "last" if i == num - 1 else "mid2" if i == num - 3 else "mid"
+            seen, left = magnitudes(kind, r, v)
+            most[kind] = max(most.get(kind, 0), seen)
+            v = left if kind in ("first", "last") else B  # a column factor ends the passes between
+        assert v <= LIFTED_MAX
+    for log_n in range(8, 13):
+        r1, r2 = (log_n + 1) // 2, log_n // 2
+        seen, v = magnitudes("first", r1, 1.0)
+        assert seen <= 2 * B + 6
+        seen, v = magnitudes("col_last", r2, v)
+        most["col_last"] = max(most.get("col_last", 0), seen)
+        assert v <= LIFTED_MAX
+    assert most["first"] <= 2 * B + 6 and most["mid"] <= 2 * B + 6 and most["last"] <= 2 * B + 6
+    assert 3 * B <= most["mid2"] <= VALUE_MAX and 3 * B <= most["col_last"] <= VALUE_MAX
+
+
+@pytest.mark.parametrize("field", FIELDS)
+def test_products_and_reductions_at_the_largest_values(field):
+    p = g.MODULI[field]
+    limit = VALUE_MAX * p
+    assert DIGITS_MAX == (TOP - 1) - OFFSET and limit <= DIGITS_MAX
+    assert sum(d << (8 * k) for k, d in enumerate(digits(limit))) == limit
+    assert sum(d << (8 * k) for k, d in enumerate(digits(-limit))) == -limit
+    assert LIFT > LIFTED_MAX and (LIFT + LIFTED_MAX) * p < TOP
+    rng = random.Random(field + 300)
+    for y in [limit, -limit, limit - 1, 3 * 6144 * p, -3 * 6144 * p] + [rng.randrange(limit // 2, limit) for _ in range(4)]:
+        assert abs(reduced(y, p)) <= 0.52 * p and (reduced(y, p) - y) % p == 0
+        for w in (1, p - 1, p // 2, p // 2 + 1, rng.randrange(p)):
+            t = product(y, w, p)
+            assert (t - y * w) % p == 0 and abs(t) <= 6144 * p + (96 * 128 * p >> 15)
