@@ -377,14 +377,15 @@ struct F753 {
             r.v[i] = __builtin_addc(a.v[i], d[i], c, &c);
         return r;
     }
-    // x mod p for x < 2^767: a quotient estimate from the top 96 bits in
+    // x mod p for any x < 2^768: a quotient estimate from the top 96 bits in
     // double precision, q_est in {q - 1, q}, then one conditional subtraction
     __device__ __forceinline__ static E753 canon(const E753 &x)
     {
         constexpr double TWO32 = 4294967296.0;
         constexpr double P_TOP = ((double)P::MOD[23] * TWO32 + (double)P::MOD[22]) * TWO32 + (double)P::MOD[21];
         const double x_top = ((double)x.v[23] * TWO32 + (double)x.v[22]) * TWO32 + (double)x.v[21];
-        // x_top / P_TOP is x/p to within a relative 2^-50; x/p < 2^15
+        // x_top / P_TOP is x/p to within a relative 2^-50; x/p < 2^15.2, so
+        // the 2^-40 takes off more than that and less than 2^-24 in all
         const uint32_t q = (uint32_t)(x_top * ((1.0 - 0x1p-40) / P_TOP));
         uint32_t r[24];
         uint64_t carry = 0;

@@ -327,3 +327,24 @@ def test_products_and_reductions_at_the_largest_values(field):
         for w in (1, p - 1, p // 2, p // 2 + 1, rng.randrange(p)):
             t = product(y, w, p)
             assert (t - y * w) % p == 0 and abs(t) <= 6144 * p + (96 * 128 * p >> 15)
+
+
+@pytest.mark.parametrize("field", FIELDS)
+def test_canon_covers_every_768_bit_value(field):
+    """F753::canon: the quotient estimate in double precision is the quotient
+    or one less, up to the lifted values of the last passes and to 2^768."""
+    p = g.MODULI[field]
+    two32 = 4294967296.0
+    limb = lambda v, i: float((v >> (32 * i)) & 0xFFFFFFFF)
+    top = lambda v: (limb(v, 23) * two32 + limb(v, 22)) * two32 + limb(v, 21)
+    factor = (1.0 - 2.0 ** -40) / top(p)
+    rng = random.Random(field + 400)
+    xs = [TOP - 1, TOP - 2, (LIFT + LIFTED_MAX) * p, 1 << 767, (1 << 767) - 1]
+    for _ in range(4000):
+        k = rng.randrange(1, TOP // p + 1)
+        xs += [k * p - 1, k * p, k * p + 1]
+    for k in list(range(1, 40)) + list(range(TOP // p - 40, TOP // p + 1)):
+        xs += [k * p - 1, k * p, k * p + 1]
+    for x in xs:
+        q = int(top(x) * factor)
+        assert x // p - 1 <= q <= x // p, x
