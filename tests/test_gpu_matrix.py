@@ -241,3 +241,36 @@ def test_largest_matrix_passes_match_vector_kernels(log_n):
             g.tuning_load(shipped)  # the default routes again
         assert np.array_equal(got, want), (log_n, inverse)
         del got, want
+
+
+def test_table_lines_on_the_vector_kernels():
+    """Every 753-bit line of the shipped table, of transforms alone and in
+    batches, set explicitly: the vector kernels run it, bit-identical to the
+    library's own choice (elsewhere against the oracle)."""
+    shipped = os.path.join(os.path.dirname(g.library_path), "tuning.txt")
+    lines = []
+    for line in open(shipped):
+        tok = [t for t in line.split("#", 1)[0].split() if t != "batch"]
+        if tok and int(tok[0]) != g.FIELD_FP32:
+            lines.append((int(tok[0]), int(tok[1]), [tuple(map(int, t.split(","))) for t in tok[2:]]))
+    assert len(lines) >= 25
+    for field, log_n, sched in sorted(lines):
+        print("vector schedule", field, log_n, sched, flush=True)
+        x = operands(field, log_n, 0x7AB + log_n)
+        want = {}
+        try:
+            g.tuning_clear()
+            g.tuning_load(shipped)
+            for inverse in (False, True):
+                plan = g.Plan(field, log_n, inverse=inverse)
+                want[inverse] = run(plan, x, in_place=False)
+                plan.close()
+            g.tuning_set(field, log_n, sched)
+            for inverse in (False, True):
+                plan = g.Plan(field, log_n, inverse=inverse)
+                assert plan.num_passes == len(sched)
+                assert np.array_equal(run(plan, x, in_place=False), want[inverse]), (field, log_n, sched, inverse)
+                plan.close()
+        finally:
+            g.tuning_clear()
+            g.tuning_load(shipped)
