@@ -5,6 +5,9 @@
 
 namespace gsn {
 
+// the smallest radix compiled as a last pass (matrix_passes' schedules end in
+// no smaller one)
+constexpr int DENSE_LAST = 5;
 // radices compiled, and columns of a block
 constexpr bool dense_supported(const PassCfg &c)
 {

@@ -249,10 +249,13 @@ template <class F, int LOG_R, int KS>
 static void launch_r(const PassJob<F> &job, bool last, uint32_t count, hipStream_t st)
 {
     const dim3 grid((1u << (job.a.log_n - 8)) * KS, count), block(256);
-    if (last)
-        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, true>), grid, block, 0, st, job.a);
-    else
-        hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, false>), grid, block, 0, st, job.a);
+    if constexpr (LOG_R >= DENSE_LAST) {
+        if (last) {
+            hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, true>), grid, block, 0, st, job.a);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((dense753_kernel<F, LOG_R, KS, false>), grid, block, 0, st, job.a);
 }
 template <class F>
 void launch_dense753(const PassJob<F> &job, bool last, uint32_t count, hipStream_t st)

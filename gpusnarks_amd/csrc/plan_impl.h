@@ -127,7 +127,7 @@ struct PlanImpl final : PlanBase {
         num_passes = (int)cfg.size();
         workspace_buffers = schedule_buffers(cfg);
         for (const PassCfg &c : cfg)
-            if (!pass_supported<F>(c))
+            if (!pass_supported<F>(c) || (c.kind == MAT_DENSE && &c == &cfg.back() && c.log_r < DENSE_LAST))
                 return set_error(GSN_ERR_INVALID_ARGUMENT, "no kernel for the pass configuration");
         scale = make_tw(H((uint32_t)n).mul_inv());
         if (log_n == 0)
