@@ -57,6 +57,10 @@ struct BatchMemory {
 
 // Which schedules the items of a batch take together.
 std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count);
+// A server's cached plan: when it is first built, so is the one of the other
+// schedule that the size takes in waves of another load, and no later request
+// waits for tables.
+int served_plan(PlanBase **out, const gsn_batch_item &it, PlanUse use);
 // Workspace bytes a batch of these items needs (256-byte aligned slices).
 size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count);
 // Builds the schedule.

@@ -165,6 +165,19 @@ std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count)
     return uses;
 }
 
+int served_plan(PlanBase **out, const gsn_batch_item &it, PlanUse use)
+{
+    bool created = false;
+    GSN_TRY(cached_plan(out, it.field, it.log_n, it.omega, it.inverse, use, &created));
+    const PlanUse other = use == FUSED ? FUSED_FEW : FUSED;
+    if (!created || choose_passes(it.field, it.log_n, other) == choose_passes(it.field, it.log_n, use))
+        return GSN_OK;
+    PlanBase *unused = nullptr;
+    if (cached_plan(&unused, it.field, it.log_n, it.omega, it.inverse, other) != GSN_OK)
+        (void)hipGetLastError();  // a wave that needs it says so
+    return GSN_OK;
+}
+
 size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count)
 {
     const std::vector<PlanUse> uses = batch_uses(items, count);
@@ -190,7 +203,8 @@ int build_batch(BatchImpl &b, const gsn_batch_item *items, size_t count, int use
         const gsn_batch_item &it = items[i];
         if (!it.d_in || !it.d_out)
             return set_error(GSN_ERR_INVALID_ARGUMENT, "batch item " + std::to_string(i) + " has a NULL buffer");
-        GSN_TRY(cached_plan(&plans[i], it.field, it.log_n, it.omega, it.inverse, uses[i]));
+        GSN_TRY(mem.alloc ? served_plan(&plans[i], it, uses[i])
+                          : cached_plan(&plans[i], it.field, it.log_n, it.omega, it.inverse, uses[i]));
         const size_t eb = element_bytes(it.field);
         const size_t n = (size_t)1 << it.log_n;
         const int nbuf = plans[i]->workspace_buffers;

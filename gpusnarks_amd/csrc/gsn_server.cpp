@@ -154,7 +154,7 @@ int enqueue_single_t(PlanBase *base, const gsn_batch_item &it, Wave *w, hipStrea
 int enqueue_single(const gsn_batch_item &it, Wave *w, hipStream_t s)
 {
     PlanBase *p = nullptr;
-    GSN_TRY(cached_plan(&p, it.field, it.log_n, it.omega, it.inverse, FUSED));
+    GSN_TRY(served_plan(&p, it, FUSED));
     switch (it.field) {
     case GSN_FIELD_FP32: return enqueue_single_t<GSN_FIELD_FP32>(p, it, w, s);
     case GSN_FIELD_MNT4753_FR: return enqueue_single_t<GSN_FIELD_MNT4753_FR>(p, it, w, s);

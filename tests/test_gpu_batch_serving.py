@@ -123,3 +123,36 @@ def test_server_admission_budget():
         srv.wait(t)
         assert np.array_equal(out, want[k])
     srv.close()
+
+
+@pytest.mark.parametrize("log_n", [16, 17])
+def test_server_builds_the_tables_of_either_schedule_at_first(log_n):
+    """2^15 to 2^17 take one of two schedules in a wave, by its load.  After one
+    request alone, the plan for the other is there: a batch that needs it is
+    created in less than half the time of one with a root not yet seen."""
+    field = g.FIELD_MNT6753_FR
+    p, n = g.MODULI[field], 1 << log_n
+    rep = sum(int(v) << (32 * i) for i, v in enumerate(np.asarray(g.root_of_unity(field, log_n)).reshape(-1)))
+    w, one = rep * pow(1 << 768, -1, p) % p, 1 << 768
+
+    def root(k):
+        v = pow(w, k, p) * one % p
+        return np.array([(v >> (32 * i)) & 0xFFFFFFFF for i in range(24)], dtype=np.uint32)
+
+    x = synth.uniform_residues(0x5E7 + log_n, n, p, 24)
+    d_in, d_out = g.DeviceArray.from_numpy(x), g.DeviceArray(x.nbytes)
+
+    def creation(omega):
+        t = time.perf_counter()
+        batch = g.Batch([(field, log_n, False, d_in.ptr, d_out.ptr, omega)], use_graph=False)
+        t = time.perf_counter() - t
+        assert batch.num_launches == 2  # the vector kernels
+        batch.close()
+        return t
+
+    srv = g.Server(hbm_budget_bytes=1 << 28)
+    say("server request", log_n)
+    srv.wait(srv.submit_device(field, log_n, d_in.ptr, d_out.ptr, omega=root(3)))
+    srv.close()
+    fresh = min(creation(root(k)) for k in (5, 7, 9))
+    assert creation(root(3)) < fresh / 2
