@@ -176,7 +176,8 @@ def write_table(results, path, keep_from=None):
     sizes and the batch lines as the existing table (`keep_from`, else `path`)
     has them."""
     lines = ["# field log_n  log_r,log_w,log_e per pass  (written by gpusnarks_amd.autotune)",
-             "# 'batch field log_n ...': the schedule of transforms fused into batches, where it differs"]
+             "# 'batch field log_n ...': the schedule of transforms fused into batches, where it differs",
+             "# the vector kernels' schedules; 753-bit sizes on the matrix cores keep a line to be reported"]
     rows = kept_lines(keep_from or path, results)
     for (field, log_n), (sched, ms, ms_default) in results.items():
         if sched is None:

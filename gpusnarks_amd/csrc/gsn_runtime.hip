@@ -126,8 +126,9 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
 // Others: passes of matrix753_kernels.h.  Radices of 2^4 .. 2^6 in tiles of
 // 32 columns, the first and the last at least 2^5 (their columns are k1 and
 // jP): three passes from 2^15, four from 2^19 to 2^24.  Where the line lies,
-// matrix against vector: 2^16 68 / 60 us, 2^17 79 / 76, 2^18 99 / 126, 2^19
-// 136 / 249, 2^20 285 / 515, 2^22 1210 / 2280: a transform of 2^16 or 2^17
+// matrix against vector, run back to back (tables cached; 2^18 with cold tables
+// 114 / 129): 2^16 68 / 60 us, 2^17 79 / 76, 2^18 99 / 126, 2^19 136 / 249, 2^20
+// 285 / 515, 2^22 1210 / 2280: a transform of 2^16 or 2^17
 // leaves most of the chip without a tile of 2^11.  Batches fill it, so there
 // everything from 2^15 goes this way (64 ragged transforms: 986 us; 998 with
 // 2^14 too, 1031 from 2^16, 1248 with none below 2^18), except the few that
