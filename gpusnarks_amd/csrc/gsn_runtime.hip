@@ -486,67 +486,61 @@ static int build_tables_753(Plan &plan, const H &w, unsigned log_n, size_t n)
     plan.step_nrec.assign(P_, 0);
     unsigned log_ns = 0;
     if (mat) {
-        const bool dense = plan.cfg[0].kind == MAT_DENSE;
-        const auto r = [&](size_t i) { return (unsigned)plan.cfg[i].log_r; };
-        // a pass's matrices are those of the first one with the same radix and
-        // (not dense, from the second pass on) the same one before it
-        plan.mat_share.resize(P_);
-        for (size_t i = 0; i < P_; ++i) {
-            size_t own = dense || i == 0 ? 0 : 1;
-            while (r(own) != r(i) || (!dense && i > 0 && r(own - 1) != r(i - 1)))
-                ++own;
-            plan.mat_share[i] = (int)own;
-        }
-        const auto owns = [&](size_t i) { return plan.mat_share[i] == (int)i; };
-        const auto between = [&](size_t i) { return i > 0 && i + 1 < P_; };
-        // entries of table k of pass i: folded, column and fixed matrices, or
-        // (dense) matrices and records
-        const auto entries = [&](size_t i, int k, unsigned before) -> size_t {
-            const unsigned g = i ? r(i - 1) : 0u;
-            if (dense)
-                return k == 0 ? (owns(i) ? (size_t)1 << r(i) : 0)
-                              : k == 1 && i + 1 < P_ ? (size_t)1 << (before + r(i) + r(i + 1)) : 0;
-            switch (k) {
-            case 0: return owns(i) ? (((size_t)1 << r(i)) - 1) << g : 0;
-            case 1: return between(i) ? (size_t)1 << (g + r(P_ - 1)) : 0;
-            default: return between(i) && i + 2 < P_ ? (size_t)2 << (g + r(2)) : 0;
-            }
-        };
-        std::vector<size_t> at(3 * P_ + 1, 0);
-        for (size_t i = 0; i < P_; log_ns += r(i), ++i)
-            for (int k = 0; k < 3; ++k) {
-                const size_t bytes = entries(i, k, log_ns) * (dense && k == 1 ? sizeof(TW753) : (size_t)MAT_BYTES);
-                at[3 * i + k + 1] = at[3 * i + k] + ((bytes + 255) & ~(size_t)255);
-            }
-        GSN_TRY(plan.mat_buf.alloc(at.back()));
         plan.mat_tabs.resize(3 * P_);
-        for (size_t x = 0; x < 3 * P_; ++x)
-            plan.mat_tabs[x] = at[x + 1] > at[x] ? (char *)plan.mat_buf.ptr + at[x] : nullptr;
-        log_ns = 0;
-        for (size_t i = 0; i < P_; log_ns += r(i), ++i) {
-            void *const *t = &plan.mat_tabs[3 * i];
-            const unsigned g = i ? r(i - 1) : 0u;
-            if (dense) {
+        plan.mat_share.resize(P_);
+        const auto build = [&](DeviceBuffer &b, size_t entries, bool fold, unsigned log_y, uint64_t mul, uint64_t add,
+                               bool pair, const TW753 *scale) {
+            GSN_TRY(b.alloc(entries * MAT_BYTES));
+            launch_build_mat753<F>((uint4 *)b.ptr, (uint32_t)entries, fold, dhi, dlo, h, log_n, log_y, mul, add, pair,
+                                   scale, 0);
+            return hip_status(hipGetLastError(), "matrix table launch");
+        };
+        if (plan.cfg[0].kind == MAT_DENSE) {
+            for (size_t i = 0; i < P_; ++i) {
+                const unsigned r = (unsigned)plan.cfg[i].log_r;
+                size_t own = 0;
+                while (plan.cfg[own].log_r != (int)r)
+                    ++own;
+                plan.mat_share[i] = (int)own;
+                log_ns += r;
+                DeviceBuffer &mat = plan.mat_tabs[3 * i], &rec = plan.mat_tabs[3 * i + 1];
+                if (own == i)
+                    GSN_TRY(mat.alloc((size_t)MAT_BYTES << r));
+                unsigned next = 0;
+                if (i + 1 < P_) {
+                    next = (unsigned)plan.cfg[i + 1].log_r;
+                    GSN_TRY(rec.alloc(sizeof(TW753) << (log_ns + next)));
+                }
                 // n^-1 on the first pass's records
-                launch_build_dense753<F>((uint4 *)t[0], r(i), (TW753 *)t[1], log_ns + r(i), t[1] ? r(i + 1) : 0u, dhi,
-                                         dlo, h, log_n, i == 0 && plan.inverse ? &plan.scale : nullptr, 0);
-            } else {
-                const auto build = [&](int k, bool fold, unsigned log_y, uint64_t mul, uint64_t add, bool pair,
-                                       const TW753 *scale) {
-                    if (t[k])
-                        launch_build_mat753<F>((uint4 *)t[k], (uint32_t)entries(i, k, log_ns), fold, dhi, dlo, h,
-                                               log_n, log_y, mul, add, pair, scale, 0);
-                };
-                build(0, true, g, 0, 0, false, nullptr);
-                // column factors w_n^(jP k(i-1) N1..N(i-2)); n^-1 on the first
-                build(1, false, r(P_ - 1), (uint64_t)1 << (log_ns - g), 0, false,
-                      i == 1 && plan.inverse ? &plan.scale : nullptr);
-                // the pair (1, 3)
-                if (t[2])
-                    build(2, false, r(2), (uint64_t)1 << r(P_ - 1), n >> (g + 1), true, nullptr);
+                launch_build_dense753<F>((uint4 *)mat.ptr, r, (TW753 *)rec.ptr, log_ns, next, dhi, dlo, h, log_n,
+                                         i == 0 && plan.inverse ? &plan.scale : nullptr, 0);
+                GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
             }
-            GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
+            return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
         }
+        const unsigned rp = (unsigned)plan.cfg[P_ - 1].log_r;
+        for (size_t i = 0; i < P_; ++i) {
+            const unsigned r = (unsigned)plan.cfg[i].log_r, g = i ? (unsigned)plan.cfg[i - 1].log_r : 0u;
+            size_t own = i;
+            for (size_t k = 1; k < i; ++k)
+                if (plan.cfg[k].log_r == (int)r && plan.cfg[k - 1].log_r == (int)g)
+                    own = std::min(own, k);
+            plan.mat_share[i] = (int)own;
+            if (own == i)
+                GSN_TRY(build(plan.mat_tabs[3 * i], (((size_t)1 << r) - 1) << g, true, g, 0, 0, false, nullptr));
+            if (i > 0 && i < P_ - 1) {
+                // column factors w_n^(jP k(i-1) N1..N(i-2)); n^-1 on the first
+                GSN_TRY(build(plan.mat_tabs[3 * i + 1], (size_t)1 << (g + rp), false, rp,
+                              (uint64_t)1 << (log_ns - g), 0, false, i == 1 && plan.inverse ? &plan.scale : nullptr));
+                if (i + 2 < P_) {  // the pair (1, 3)
+                    const unsigned r3 = (unsigned)plan.cfg[2].log_r;
+                    GSN_TRY(build(plan.mat_tabs[3 * i + 2], (size_t)2 << (g + r3), false, r3, (uint64_t)1 << rp,
+                                  n >> (g + 1), true, nullptr));
+                }
+            }
+            log_ns += r;
+        }
+        GSN_TRY(hip_status(hipGetLastError(), "matrix table launch"));
         return hip_status(hipStreamSynchronize(nullptr), "matrix tables");
     }
     for (size_t i = 0; i < P_; ++i) {

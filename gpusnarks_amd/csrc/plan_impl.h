@@ -106,15 +106,14 @@ struct PlanImpl final : PlanBase {
     std::vector<uint32_t> step_nrec;
     // 753-bit matrix passes, per pass: folded, column and fixed matrices, or
     // (dense) matrices and the next pass's records; a pass whose first ones
-    // equal another's has the owner in mat_share.  All in one allocation.
-    DeviceBuffer mat_buf;
-    std::vector<void *> mat_tabs;
+    // equal another's has the owner in mat_share
+    std::vector<DeviceBuffer> mat_tabs;
     std::vector<int> mat_share;
     // 32-bit, per pass: column table w_R^x (x < R) and pass table in units
     // of w_{Ns R} -- direct, or hi/lo halves of a two-level split
     std::vector<DeviceBuffer> col_tabs, pass_tabs, pass_los, pass_as;
     std::vector<uint32_t> pass_lo_bits;
-    DeviceBuffer scratch;  // the workspace buffers, each from a 256-byte boundary
+    DeviceBuffer scratch[2];
     tw scale{};
 
     static tw make_tw(const H &w);
@@ -133,20 +132,18 @@ struct PlanImpl final : PlanBase {
         if (log_n == 0)
             return GSN_OK;
         GSN_TRY(build_tables(w, n));
-        device_bytes = mat_buf.bytes;
-        for (auto *v : {&col_tabs, &pass_tabs, &pass_los, &pass_as, &step_tabs})
+        device_bytes = 0;
+        for (auto *v : {&col_tabs, &pass_tabs, &pass_los, &pass_as, &step_tabs, &mat_tabs})
             for (auto &b : *v)
                 device_bytes += b.bytes;
         return GSN_OK;
     }
 
-    // ws: the workspace of `count` transforms side by side
-    int ensure_scratch(size_t count, void *(&ws)[2])
+    int ensure_scratch()
     {
-        const size_t one = ((count << log_n) * sizeof(elem) + 255) & ~(size_t)255;
-        GSN_TRY(scratch.alloc((size_t)workspace_buffers * one));
-        ws[0] = scratch.ptr;
-        ws[1] = workspace_buffers > 1 ? (char *)scratch.ptr + one : nullptr;
+        const size_t bytes = ((size_t)1 << log_n) * sizeof(elem);
+        for (int i = 0; i < workspace_buffers; ++i)
+            GSN_TRY(scratch[i].alloc(bytes));
         return GSN_OK;
     }
 
@@ -190,15 +187,15 @@ struct PlanImpl final : PlanBase {
                 a.lo_bits = pass_lo_bits[i];
                 a.pass_shift = 0;
             } else if (dense) {
-                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]];
-                a.tw_pass = (const tw *)mat_tabs[3 * i + 1];
+                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]].ptr;
+                a.tw_pass = (const tw *)mat_tabs[3 * i + 1].ptr;
                 a.log_np = i + 1 < P ? (uint32_t)cfg[i + 1].log_r : 0u;
             } else if (mat) {
                 // digits of this pass, those after it in the index and the
                 // one before it, as matrix753_kernels.h describes them
-                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]];
-                a.tw_pass = (const tw *)mat_tabs[3 * i + 1];
-                a.tw_pass_a = (const tw *)mat_tabs[3 * i + 2];
+                a.tw_col = (const tw *)mat_tabs[3 * mat_share[i]].ptr;
+                a.tw_pass = (const tw *)mat_tabs[3 * i + 1].ptr;
+                a.tw_pass_a = (const tw *)mat_tabs[3 * i + 2].ptr;
                 a.log_s = log_n - log_ns - (uint32_t)c.log_r;
                 a.log_g = i == 0 ? 0u : (uint32_t)cfg[i - 1].log_r;
                 a.log_np = (uint32_t)cfg[P - 1].log_r;
@@ -240,10 +237,9 @@ struct PlanImpl final : PlanBase {
             launch_scale<F>((const elem *)in, (elem *)out, scale, n, 0, s);
             return hip_status(hipGetLastError(), "scale_kernel launch");
         }
-        void *ws[2];
-        GSN_TRY(ensure_scratch(1, ws));
+        GSN_TRY(ensure_scratch());
         std::vector<PassJob<F>> jobs;
-        make_jobs(in, out, ws[0], ws[1], jobs);
+        make_jobs(in, out, scratch[0].ptr, scratch[1].ptr, jobs);
         for (size_t i = 0; i < jobs.size(); ++i) {
             launch_pass<F>(jobs[i], cfg[i], s);
             GSN_TRY(hip_status(hipGetLastError(), "ntt pass launch"));
@@ -257,10 +253,10 @@ struct PlanImpl final : PlanBase {
     int execute_two(const void *in, void *out, hipStream_t s)
     {
         if constexpr (!IS32) {
-            void *ws[2];
-            GSN_TRY(ensure_scratch(2, ws));
+            for (int i = 0; i < workspace_buffers; ++i)
+                GSN_TRY(scratch[i].alloc(((size_t)2 << log_n) * sizeof(elem)));
             std::vector<PassJob<F>> jobs;
-            make_jobs(in, out, ws[0], ws[1], jobs);
+            make_jobs(in, out, scratch[0].ptr, scratch[1].ptr, jobs);
             for (size_t i = 0; i < jobs.size(); ++i) {
                 launch_dense753<F>(jobs[i], i + 1 == jobs.size(), 2, s);
                 GSN_TRY(hip_status(hipGetLastError(), "ntt pass launch"));
