@@ -579,7 +579,7 @@ def main():
     args = ap.parse_args()
     set_settle_ms(args.settle_ms)
     if args.gpus != 1:
-        print("bench.py measures one GPU: this build has no multi-GPU path (the box has one MI355X); "
+        print("bench.py measures one GPU: this build has no multi-GPU path (one MI355X); "
               "run with --gpus 1", file=sys.stderr)
         sys.exit(2)
 

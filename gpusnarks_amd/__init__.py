@@ -38,7 +38,7 @@ MODULI = {
 }
 
 _PKG = os.path.dirname(os.path.abspath(__file__))
-# $GSN_LIBRARY selects another build of the library (same-box comparisons)
+# $GSN_LIBRARY selects another build of the library (comparisons on one GPU)
 library_path = os.environ.get("GSN_LIBRARY") or os.path.join(_PKG, "libgpusnarks.so")
 
 _u32p = ctypes.POINTER(ctypes.c_uint32)

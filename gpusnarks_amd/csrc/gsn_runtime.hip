@@ -119,7 +119,7 @@ std::vector<PassCfg> default_passes(int field, unsigned L)
 //
 // Alone, 2^10 .. 2^15: dense passes (dense753.hip), whose work grows as n R
 // and which need 32 columns.  Against the vector kernels, with other radices
-// in brackets, time on one box: 2^10 16 / 35 us, 2^11 18 / 40, 2^12 20 / 41
+// in brackets, times on one card: 2^10 16 / 35 us, 2^11 18 / 40, 2^12 20 / 41
 // (three passes 22), 2^13 23 / 44 (2^7 2^6 25), 2^14 26 / 48 (2^7 2^7 30),
 // 2^15 36 / 57 (the passes below 50), 2^16 60-64 / 60.
 //
