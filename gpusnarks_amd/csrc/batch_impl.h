@@ -57,9 +57,9 @@ struct BatchMemory {
 
 // Which schedules the items of a batch take together.
 std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count);
-// A server's cached plan: when it is first built, so is the one of the other
-// schedule that the size takes in waves of another load, and no later request
-// waits for tables.
+// A server's cached plan; the one of the other schedule that the size may take,
+// in waves of another load, is built with it, so that no later request waits
+// for tables (whoever else has built either).
 int served_plan(PlanBase **out, const gsn_batch_item &it, PlanUse use);
 // Workspace bytes a batch of these items needs (256-byte aligned slices).
 size_t batch_workspace_bytes(const gsn_batch_item *items, size_t count);

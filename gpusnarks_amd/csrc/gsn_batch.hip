@@ -167,10 +167,11 @@ std::vector<PlanUse> batch_uses(const gsn_batch_item *items, size_t count)
 
 int served_plan(PlanBase **out, const gsn_batch_item &it, PlanUse use)
 {
-    bool created = false;
-    GSN_TRY(cached_plan(out, it.field, it.log_n, it.omega, it.inverse, use, &created));
+    GSN_TRY(cached_plan(out, it.field, it.log_n, it.omega, it.inverse, use));
     const PlanUse other = use == FUSED ? FUSED_FEW : FUSED;
-    if (!created || choose_passes(it.field, it.log_n, other) == choose_passes(it.field, it.log_n, use))
+    // a field whose sizes end at 2^15 fills its matrix passes (batch_uses)
+    if (it.log_n < 15 || it.log_n > 17 || two_adicity(it.field) <= 15 ||
+        choose_passes(it.field, it.log_n, other) == choose_passes(it.field, it.log_n, use))
         return GSN_OK;
     PlanBase *unused = nullptr;
     if (cached_plan(&unused, it.field, it.log_n, it.omega, it.inverse, other) != GSN_OK)

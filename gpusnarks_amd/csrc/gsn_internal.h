@@ -84,9 +84,7 @@ int staged_d2h(void *host, const void *dev, size_t bytes, hipStream_t st);
 int create_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use = ALONE);
 void clear_schedules();
 void clear_plan_cache();
-// *created: whether this call built it
-int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use = ALONE,
-                bool *created = nullptr);
+int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use = ALONE);
 
 }  // namespace gsn
 

@@ -658,10 +658,8 @@ void clear_plan_cache()
     g_plan_cache.clear();
 }
 
-int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use, bool *created)
+int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, int inverse, PlanUse use)
 {
-    if (created)
-        *created = false;
     std::string key(16, '\0');
     std::memcpy(&key[0], &field, 4);
     std::memcpy(&key[4], &log_n, 4);
@@ -679,8 +677,6 @@ int cached_plan(PlanBase **out, int field, unsigned log_n, const void *omega, in
     GSN_TRY(create_plan(&p, field, log_n, omega, inverse, use));
     g_plan_cache[key].reset(p);
     *out = p;
-    if (created)
-        *created = true;
     return GSN_OK;
 }
 

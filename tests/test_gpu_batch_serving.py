@@ -150,9 +150,15 @@ def test_server_builds_the_tables_of_either_schedule_at_first(log_n):
         batch.close()
         return t
 
+    # a batch has built the plan of a full wave for the second root already
+    batch = g.Batch([(field, log_n, False, d_in.ptr, d_out.ptr, root(11))] * 8, use_graph=False)
+    assert batch.num_launches == 3
+    batch.close()
     srv = g.Server(hbm_budget_bytes=1 << 28)
     say("server request", log_n)
-    srv.wait(srv.submit_device(field, log_n, d_in.ptr, d_out.ptr, omega=root(3)))
+    for k in (3, 11):
+        srv.wait(srv.submit_device(field, log_n, d_in.ptr, d_out.ptr, omega=root(k)))
     srv.close()
     fresh = min(creation(root(k)) for k in (5, 7, 9))
     assert creation(root(3)) < fresh / 2
+    assert creation(root(11)) < fresh / 2
